@@ -100,6 +100,40 @@ __device__ __forceinline__ int solve_3x3_gepp(const G* a, G* b, G* minpiv = null
   return 0;
 }
 
+// solve_3x3_gepp in double with the rows picked by selects: a wave's lanes
+// pivot differently, and as branches every lane sat through up to three
+// versions of the first elimination and two of the second (five rows of
+// divisions instead of two).  The operations on the picked rows are the
+// reference's, so the solution has its bits.  b is overwritten in any case; a
+// caller discards it when the result is 1.
+__device__ __forceinline__ int solve_3x3_gepp_select(const double* a, double* b) {
+  // copies: a conditional over array elements would pick between addresses
+  // and put the array in scratch memory
+  const double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3], a4 = a[4], a5 = a[5], a6 = a[6],
+               a7 = a[7], a8 = a[8], b0 = b[0], b1 = b[1], b2 = b[2];
+  const double aa0 = fabs(a0), aa1 = fabs(a1), aa2 = fabs(a2);
+  const bool p0 = aa0 >= aa1 && aa0 >= aa2;
+  const bool p1 = !(aa0 >= aa1) && aa1 >= aa2;  // neither: row 2
+  const bool p2 = !(p0 || p1);
+  const double l0 = p0 ? a0 : (p1 ? a1 : a2), l1 = p0 ? a3 : (p1 ? a4 : a5),
+               l2 = p0 ? a6 : (p1 ? a7 : a8), bl = p0 ? b0 : (p1 ? b1 : b2);
+  const double m0 = p0 ? a1 : a0, m1 = p0 ? a4 : a3, m2 = p0 ? a7 : a6, mb = p0 ? b1 : b0;
+  const double n0 = p2 ? a1 : a2, n1 = p2 ? a4 : a5, n2 = p2 ? a7 : a8, nb = p2 ? b1 : b2;
+  const double f1 = m0 / l0, f2 = n0 / l0;
+  const double lm1 = m1 - f1 * l1, lm2 = m2 - f1 * l2, ln1 = n1 - f2 * l1, ln2 = n2 - f2 * l2;
+  const double bm = mb - f1 * bl, bn = nb - f2 * bl;
+  const bool pm = fabs(lm1) >= fabs(ln1);
+  const double x1 = pm ? lm1 : ln1, x2 = pm ? lm2 : ln2, xb = pm ? bm : bn;
+  const double y1 = pm ? ln1 : lm1, y2 = pm ? ln2 : lm2, yb = pm ? bn : bm;
+  const double g = y1 / x1;
+  const double q2 = y2 - g * x2;
+  const double s2 = (yb - g * xb) / q2;
+  const double s1 = (xb - x2 * s2) / x1;
+  const double s0 = (bl - s1 * l1 - s2 * l2) / l0;
+  b[0] = s0; b[1] = s1; b[2] = s2;
+  return fabs(l0) <= DBL_EPSILON || fabs(x1) < DBL_EPSILON ? 1 : 0;
+}
+
 // The FP32 Newton step's 3x3 solve (column-major a), by the adjugate: x =
 // adj(a) b / det(a), with no data-dependent branch, so that a wave's lanes
 // do not each take their own pivoting path.  Returns 1 without a solution
@@ -591,6 +625,117 @@ __device__ int nsn_newton_std_fp32(const LocalProblem<T>& lp, T* r, const LocalP
   return 1;
 }
 
+// sqrt(x) * s < t, the root taken only where the squares do not decide: the
+// test of a Newton iterate is mostly orders of magnitude off its threshold.
+// x s^2 and t^2 carry a few ulp each, so 1e-9 apart they order as the rounded
+// sqrt(x) * s and t do (t^2 > 1e-290 keeps the products clear of underflow;
+// s is 1 or at most 1 / DBL_EPSILON).  NaNs take the exact test.
+__device__ __forceinline__ bool root_below(double x, double s, double t) {
+  const double t2 = t * t, y = x * s * s;
+  if (t > 0.0 && t2 > 1e-290) {
+    if (y < t2 * (1.0 - 1e-9)) return true;
+    if (y > t2 * (1.0 + 1e-9)) return false;
+  }
+  return sqrt(x) * s < t;
+}
+
+// nsn_newton's loop (onecontact...c:429-559 and 710-854) for the FP64 sweeps
+// with the STD formulation: the same operations, so the same bits, with what
+// the reference computes twice computed once:
+//   the A and B of an iteration are finished from the intermediates of the F
+//   evaluation that tested the same iterate;
+//   A's first row is (A_00, 0, 0), so A W needs no products with its zeros;
+//   the line search's directional derivative reads the Newton matrix
+//   -(A W + B) instead of forming A W + B again (each product and sum is the
+//   negative of the reference's);
+//   the residual sqrt(*F2) * *nrel and |dR| are compared by their squares
+//   (root_below); a caller that needs the residual's value takes the root.
+// The line search is the reference's (:562-708).
+__device__ inline int nsn_newton_std_fp64(const LocalProblem<double>& lp, double* r,
+                                          const LocalParams& P, double tol, const double* rho,
+                                          bool damped, double* F2, double* nrel_out) {
+  const double nq = sqrt(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
+  double nrel = 1.0;
+  if (nq > DBL_EPSILON) nrel = nrel / nq;
+  *nrel_out = nrel;
+  double dR[3] = {0.0, 0.0, 0.0}, F[3], v[3];
+  double A[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  double B[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  AcStdPoint<double> pt;
+  local_velocity<double>(lp, r, v);
+  double t = 1.0;
+  ac_std_f<double>(r, v, lp.mu, rho, F, pt);
+  *F2 = F[0] * F[0] + F[1] * F[1] + F[2] * F[2];
+  if (root_below(*F2, nrel, tol)) return 0;
+  for (int inew = 1; inew < P.newton_max_iter; ++inew) {
+    ac_std_ab<double>(pt, lp.mu, rho, A, B);
+    const double* W = lp.W;
+    double M[9];  // -(A W + B)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      M[3 * j] = (A[0] * W[3 * j] + B[3 * j]) * -1.0;
+#pragma unroll
+      for (int i = 1; i < 3; i++)
+        M[i + 3 * j] =
+            (A[i] * W[3 * j] + A[i + 3] * W[3 * j + 1] + A[i + 6] * W[3 * j + 2] + B[i + 3 * j]) *
+            -1.0;
+    }
+    dR[0] = F[0]; dR[1] = F[1]; dR[2] = F[2];
+    const int info3 = solve_3x3_gepp_select(M, dR);
+    if (info3) {
+      dR[0] = 0.0; dR[1] = 0.0; dR[2] = 0.0;
+    }
+    if (damped) {
+      if (!info3) {
+        double alpha = 1.0;
+        const double inf = 1e20;
+        double amin = 0.0, amax = inf;
+        const double q0 = 0.5 * *F2;
+        double dqdt0 = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+          dqdt0 += F[i] * -(M[i] * dR[0] + M[i + 3] * dR[1] + M[i + 6] * dR[2]);
+        for (int it = 0; it < P.ls_max_iter; it++) {
+          double rt[3];
+          AcStdPoint<double> unused;
+#pragma unroll
+          for (int i = 0; i < 3; i++) rt[i] = r[i] + alpha * dR[i];
+          local_velocity_inline<double>(lp, rt, v);
+          ac_std_f<double>(rt, v, lp.mu, rho, F, unused);
+          const double q = 0.5 * (F[0] * F[0] + F[1] * F[1] + F[2] * F[2]);
+          const double slope = (q - q0) / alpha;
+          const bool C1 = slope >= 0.9 * dqdt0;
+          const bool C2 = slope <= 0.1 * dqdt0;
+          if (C1 && C2) break;
+          if (!C1)
+            amin = alpha;
+          else
+            amax = alpha;
+          if (alpha < inf)
+            alpha = 0.5 * (amin + amax);
+          else
+            alpha = 10.0 * alpha;
+        }
+        t = alpha;
+      }
+      r[0] = r[0] + t * dR[0];
+      r[1] = r[1] + t * dR[1];
+      r[2] = r[2] + t * dR[2];
+    } else {
+      r[0] += dR[0]; r[1] += dR[1]; r[2] += dR[2];
+    }
+    local_velocity<double>(lp, r, v);
+    ac_std_f<double>(r, v, lp.mu, rho, F, pt);
+    *F2 = F[0] * F[0] + F[1] * F[1] + F[2] * F[2];
+    if (damped && info3) break;
+    if (root_below(*F2, nrel, tol)) return 0;
+    if (root_below(dR[0] * dR[0] + dR[1] * dR[1] + dR[2] * dR[2], 1.0, 10.0 * DBL_EPSILON))
+      return 1;
+    if (info3) break;
+  }
+  return 1;
+}
+
 // onecontact...c:429-559 (damped = false) and 710-854 (damped = true)
 template <typename T>
 __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P, T tol,
@@ -598,6 +743,14 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
   if constexpr (sizeof(T) == 4) {
     if (!damped && P.formulation != 1)
       return nsn_newton_std_fp32<T>(lp, r, P, tol, rho, residual);
+  }
+  if constexpr (sizeof(T) == 8) {
+    if (P.formulation != 1) {
+      double F2, nrel;
+      const int info = nsn_newton_std_fp64(lp, r, P, tol, rho, damped, &F2, &nrel);
+      *residual = sqrt(F2) * nrel;
+      return info;
+    }
   }
   const T nq = qsqrt<T>(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
   T nrel = T(1);
@@ -626,7 +779,7 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
     d[0] = F[0]; d[1] = F[1]; d[2] = F[2];
     int info3;
     if constexpr (sizeof(T) == 8) {
-      info3 = solve_3x3_gepp<T>(M, d);
+      info3 = solve_3x3_gepp_select(M, d);
     } else {
       // FP32 adjugate solve, redone in FP64 for a near-degenerate matrix
       T scale = T(0);
@@ -749,15 +902,57 @@ __device__ __forceinline__ void keep_or_discard(const LocalProblem<T>& lp, T* r,
   }
 }
 
+// The damped Newton of the hybrid solver, of whose residual it reads only
+// whether it is a number: with the STD formulation in FP64 that is whether
+// |F|^2 is one (1 / |q| is at most 1 / DBL_EPSILON), and no root is taken.
+template <typename T>
+__device__ __forceinline__ int hybrid_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
+                                             T tol, const T* rho, T* res) {
+  if constexpr (sizeof(T) == 8) {
+    if (P.formulation != 1) {
+      double nrel;
+      return nsn_newton_std_fp64(lp, r, P, tol, rho, true, res, &nrel);
+    }
+  }
+  return nsn_newton<T>(lp, r, P, tol, rho, true, res);
+}
+
 // onecontact...c:920-1015
 template <typename T>
 __device__ int hybrid_solve(const LocalProblem<T>& lp, T* r, const LocalParams& P, T tol,
                             T* rho_pli, const T* rho, T* residual) {
   int info = -1;
   T bak[3] = {r[0], r[1], r[2]};
-  T cur = compute_local_error<T>(lp, r);
-  T res = T(0);
-  if (P.hybrid_strategy == 2) {
+  T res = T(0), cur;
+  if constexpr (sizeof(T) == 8) {
+    // the starting error matters only where the Newton solution is not
+    // accepted by its own error, so it is evaluated only there
+    if (P.hybrid_strategy == 2) {
+      info = hybrid_newton<T>(lp, r, P, tol, rho, &res);
+      const T e = compute_local_error<T>(lp, r);
+      const bool number = !(isnan(res) || isinf(res));
+      if (number && e <= tol) {
+        *residual = e;
+        return info;
+      }
+      cur = compute_local_error<T>(lp, bak);
+      if (number && e <= cur) {
+        cur = e;
+        bak[0] = r[0]; bak[1] = r[1]; bak[2] = r[2];
+      } else {
+        r[0] = bak[0]; r[1] = bak[1]; r[2] = bak[2];
+      }
+      if (cur <= tol) {
+        *residual = cur;
+        return info;
+      }
+    } else {
+      cur = compute_local_error<T>(lp, r);
+    }
+  } else {
+    cur = compute_local_error<T>(lp, r);
+  }
+  if (sizeof(T) == 4 && P.hybrid_strategy == 2) {
     info = nsn_newton<T>(lp, r, P, tol, rho, true, &res);
     keep_or_discard<T>(lp, r, bak, tol, res, &cur);
     if (cur <= tol) {
@@ -771,7 +966,7 @@ __device__ int hybrid_solve(const LocalProblem<T>& lp, T* r, const LocalParams& 
     info = pli_solve<T>(lp, r, P.hybrid_max_iter, tol, rho_pli, &res);
     keep_or_discard<T>(lp, r, bak, tol, res, &cur);
     if (cur < tol) break;
-    info = nsn_newton<T>(lp, r, P, tol, rho, true, &res);
+    info = hybrid_newton<T>(lp, r, P, tol, rho, &res);
     keep_or_discard<T>(lp, r, bak, tol, res, &cur);
   }
   *residual = cur;

@@ -209,3 +209,37 @@ def test_fp32_local_solve_against_fp64(oracle, lib):
     assert worst_good < 1e-4  # measured 6.2e-6
     assert worst_err < 1e-5   # measured 6.9e-7; FP64's own is ~1e-16
     assert (i32 == 0).mean() > 0.99
+
+
+@pytest.mark.parametrize("scale", [(1.0, 1e3, 1.0), (1.0, 1.0, 1e3), (1e3, 1.0, 1e-3),
+                                   (1.0, 1.0, 0.0), (1.0, 1e-9, 1e-9)])
+@pytest.mark.parametrize("sid", [565, 551, 550])
+def test_local_solve_pivots_and_singular_blocks(oracle, lib, sid, scale):
+    """Blocks D S D whose Newton matrices pivot on each of their rows, and
+    singular or nearly singular ones (a zero or tiny scale), against the
+    oracle bit for bit."""
+    rng = np.random.default_rng(61)
+    n = 400
+    D = np.diag(scale)
+    M = rng.normal(size=(n, 3, 3))
+    S = D @ (M @ M.transpose(0, 2, 1) + 0.5 * np.eye(3)) @ D
+    q = rng.normal(size=(n, 3))
+    q[:, 0] = -abs(q[:, 0])
+    W = np.ascontiguousarray(S.transpose(0, 2, 1)).reshape(-1)
+    qf, mu, r = np.ascontiguousarray(q).reshape(-1), rng.uniform(0.1, 0.9, n), np.zeros(3 * n)
+    r[::6] = rng.uniform(0.0, 1.0, n // 2)
+    o = oracle.Options.local(sid)
+    p = local_params_from(o, sid)
+    rg, state, info = r.copy(), np.zeros(4 * n), np.zeros(n, dtype=np.int32)
+    assert lib.fc3d_hip_local_solve(n, N.dptr(W), N.dptr(qf), N.dptr(mu), N.dptr(rg), p,
+                                    N.dptr(state), 1, N.iptr(info)) == 0, capi.last_error()
+    L = oracle.load()
+    for k in range(n):
+        st = np.zeros(4)
+        w = W[9 * k:9 * k + 9].copy()
+        L.oracle_local_state_init(oracle.d(w), o.p, oracle.d(st))
+        x = r[3 * k:3 * k + 3].copy()
+        L.oracle_local_solve(oracle.d(w), oracle.d(qf[3 * k:3 * k + 3].copy()), mu[k],
+                             oracle.d(x), o.p, oracle.d(st))
+        np.testing.assert_array_equal(rg[3 * k:3 * k + 3], x, err_msg=f"contact {k}")
+        np.testing.assert_array_equal(state[4 * k:4 * k + 4], st)
