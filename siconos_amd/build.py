@@ -25,7 +25,10 @@ C_FLAGS = ["-O2", "-fPIC", "-std=gnu11", "-Wall", "-Wextra", "-Wno-unused-parame
 # the reference's C; the packed-fp32 feature is disabled on purpose.
 HIP_FLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-ffp-contract=off",
              "-fvisibility=hidden", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-             "-Wno-unused-result", "-Wno-unused-value", "-I", INC]
+             "-Wno-unused-result", "-Wno-unused-value", "-I", INC,
+             # the leading scalar arguments of a kernel arrive in registers
+             # instead of through a load at its start
+             "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 
 def _hip_flags(src):

@@ -157,9 +157,21 @@ __device__ __forceinline__ int solve_3x3_adjugate(const float* a, float* b, floa
 }
 
 // projectionOnCone.c:32-50
+// In double without branches: a wave's contacts mostly take all three ways,
+// and the selects cost less than the three exec-masked regions.
 template <typename T>
 __device__ __forceinline__ unsigned projection_on_cone(T* r, T mu) {
   const T nt = qsqrt<T>(r[1] * r[1] + r[2] * r[2]);
+  if constexpr (sizeof(T) == 8) {
+    const T r0 = r[0], r1 = r[1], r2 = r[2];
+    const bool zero = mu * nt <= -r0, inside = !zero && nt <= mu * r0;
+    const T n0 = (mu * nt + r0) / (mu * mu + T(1));
+    const T n1 = mu * n0 * r1 / nt, n2 = mu * n0 * r2 / nt;
+    r[0] = zero ? T(0) : (inside ? r0 : n0);
+    r[1] = zero ? T(0) : (inside ? r1 : n1);
+    r[2] = zero ? T(0) : (inside ? r2 : n2);
+    return zero ? 0u : (inside ? 1u : 2u);
+  }
   if (mu * nt <= -r[0]) {
     r[0] = T(0); r[1] = T(0); r[2] = T(0);
     return 0u;
@@ -625,18 +637,79 @@ __device__ int nsn_newton_std_fp32(const LocalProblem<T>& lp, T* r, const LocalP
   return 1;
 }
 
-// sqrt(x) * s < t, the root taken only where the squares do not decide: the
-// test of a Newton iterate is mostly orders of magnitude off its threshold.
-// x s^2 and t^2 carry a few ulp each, so 1e-9 apart they order as the rounded
-// sqrt(x) * s and t do (t^2 > 1e-290 keeps the products clear of underflow;
-// s is 1 or at most 1 / DBL_EPSILON).  NaNs take the exact test.
-__device__ __forceinline__ bool root_below(double x, double s, double t) {
-  const double t2 = t * t, y = x * s * s;
-  if (t > 0.0 && t2 > 1e-290) {
-    if (y < t2 * (1.0 - 1e-9)) return true;
-    if (y > t2 * (1.0 + 1e-9)) return false;
+// sqrt(x) / d < t or <= t (with `equal`), the root and the quotient taken only
+// where the squares do not decide: these tests are mostly orders of magnitude
+// off their threshold.  x and (t d)^2 carry a few ulp each, so when they are a
+// factor 1 +- 1e-9 apart they order as the rounded sides do; t d > 1e-140 and
+// x < 1e290 keep the products clear of underflow and overflow.  NaNs take the
+// exact test.  `exact` evaluates the test in the reference's operations.
+template <typename E>
+__device__ __forceinline__ bool root_test(double x, double td, E exact) {
+  const double y = td * td;
+  const bool sure = td > 1e-140 && x < 1e290 && y < 1e290;
+  const bool below = sure && x < y * (1.0 - 1e-9), above = sure && x > y * (1.0 + 1e-9);
+  if (below || above) return below;
+  return exact();
+}
+
+// ac_std_f and ac_std_ab in double without branches (a wave's contacts take
+// every way, and the quotient would sit in a branch of its own): the same
+// operations on the entries that the contact's case sets, so the same bits.
+// RV1 is cleared where the contact does not slide, which turns the sliding
+// terms into the zeros that the other cases add to (x + 0 = x); only the sign
+// of a zero can differ.  Where a value is not finite, a zero times it would
+// not be zero, and the reference's branches are taken instead.
+__device__ __forceinline__ bool ac_finite(const AcStdPoint<double>& p, const double* rho) {
+  return p.RV + fabs(p.Radius) + fabs(rho[0]) < 1e300;
+}
+
+__device__ __forceinline__ void ac_point_fp64(const double* R, const double* u, double mu,
+                                              const double* rho, double* F,
+                                              AcStdPoint<double>& p) {
+  const double RhoN = rho[0], RhoT = rho[1];
+  const double RVN = R[0] - RhoN * u[0];
+  p.RVT = R[1] - RhoT * u[1];
+  p.RVS = R[2] - RhoT * u[2];
+  p.RV = sqrt(p.RVT * p.RVT + p.RVS * p.RVS);
+  p.normal_active = RVN > 0.0;
+  p.Radius = p.normal_active ? mu * RVN : 0.0;
+  if (!ac_finite(p, rho)) {
+    ac_std_f<double>(R, u, mu, rho, F, p);
+    return;
   }
-  return sqrt(x) * s < t;
+  const bool stick = p.RV <= p.Radius;
+  const double inv = 1.0 / p.RV;
+  p.RV1 = !stick && p.Radius > 0.0 ? inv : 0.0;
+  const double F1 = R[1] - p.Radius * p.RVT * p.RV1, F2 = R[2] - p.Radius * p.RVS * p.RV1;
+  F[0] = p.normal_active ? RhoN * u[0] : R[0];
+  F[1] = stick ? RhoT * u[1] : F1;
+  F[2] = stick ? RhoT * u[2] : F2;
+}
+
+__device__ __forceinline__ void ac_jacobians_fp64(const AcStdPoint<double>& p, double mu,
+                                                  const double* rho, double* A, double* B) {
+  if (!ac_finite(p, rho)) {
+    ac_std_ab<double>(p, mu, rho, A, B);
+    return;
+  }
+  const double RhoN = rho[0], RhoT = rho[1];
+  const double RVT = p.RVT, RVS = p.RVS, Radius = p.Radius, RV1 = p.RV1;
+  const bool stick = p.RV <= Radius;
+  const double dA = stick ? RhoT : 0.0, dB = stick ? 0.0 : 1.0;
+  const double RV3 = RV1 * RV1 * RV1;
+  const double GTT = RV1 - RVT * RVT * RV3, GTS = -RVT * RVS * RV3, GSS = RV1 - RVS * RVS * RV3;
+  A[0] = p.normal_active ? RhoN : 0.0;
+  B[0] = p.normal_active ? 0.0 : 1.0;
+  A[1] = mu * RhoN * RVT * RV1;
+  A[2] = mu * RhoN * RVS * RV1;
+  A[4] = GTT * RhoT * Radius + dA;
+  A[5] = A[7] = GTS * RhoT * Radius;
+  A[8] = GSS * RhoT * Radius + dA;
+  B[1] = -mu * RVT * RV1;
+  B[2] = -mu * RVS * RV1;
+  B[4] = dB - GTT * Radius;
+  B[5] = B[7] = -GTS * Radius;
+  B[8] = dB - GSS * Radius;
 }
 
 // nsn_newton's loop (onecontact...c:429-559 and 710-854) for the FP64 sweeps
@@ -644,31 +717,47 @@ __device__ __forceinline__ bool root_below(double x, double s, double t) {
 // the reference computes twice computed once:
 //   the A and B of an iteration are finished from the intermediates of the F
 //   evaluation that tested the same iterate;
+//   the iterate a line search accepts is the point it has just evaluated (its
+//   velocity adds the same products in the same order, onecontact...c:624-626,
+//   and 1 * dR = dR), so F is not evaluated there again; only a search that
+//   runs out of trials leaves an unevaluated point;
+//   the first trial, alpha = 1, needs no quotient;
 //   A's first row is (A_00, 0, 0), so A W needs no products with its zeros;
 //   the line search's directional derivative reads the Newton matrix
 //   -(A W + B) instead of forming A W + B again (each product and sum is the
 //   negative of the reference's);
 //   the residual sqrt(*F2) * *nrel and |dR| are compared by their squares
-//   (root_below); a caller that needs the residual's value takes the root.
-// The line search is the reference's (:562-708).
+//   (root_test); a caller that needs the residual's value takes the root.
+// With one wave a SIMD every instruction takes 5.5-9 cycles and the wave sits
+// through its slowest contact's two or three iterations, so the count of
+// instructions is the time: a launch over a colour of 1000 contacts took 14.1
+// us with the reference's evaluations and branches and takes 11.9, 50k
+// contacts 20.5 -> 19.0, the 300k pile 23.1 -> 21.2.
 __device__ inline int nsn_newton_std_fp64(const LocalProblem<double>& lp, double* r,
                                           const LocalParams& P, double tol, const double* rho,
                                           bool damped, double* F2, double* nrel_out) {
   const double nq = sqrt(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
-  double nrel = 1.0;
-  if (nq > DBL_EPSILON) nrel = nrel / nq;
+  double nrel = 1.0, td = tol;
+  if (nq > DBL_EPSILON) {
+    nrel = nrel / nq;
+    td = tol * nq;
+  }
   *nrel_out = nrel;
-  double dR[3] = {0.0, 0.0, 0.0}, F[3], v[3];
+  double dR[3] = {0.0, 0.0, 0.0}, F[3] = {0.0, 0.0, 0.0}, v[3];
   double A[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double B[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   AcStdPoint<double> pt;
   local_velocity<double>(lp, r, v);
-  double t = 1.0;
-  ac_std_f<double>(r, v, lp.mu, rho, F, pt);
-  *F2 = F[0] * F[0] + F[1] * F[1] + F[2] * F[2];
-  if (root_below(*F2, nrel, tol)) return 0;
-  for (int inew = 1; inew < P.newton_max_iter; ++inew) {
-    ac_std_ab<double>(pt, lp.mu, rho, A, B);
+  ac_point_fp64(r, v, lp.mu, rho, F, pt);
+  double f2 = F[0] * F[0] + F[1] * F[1] + F[2] * F[2];
+  auto converged = [&]() {
+    return root_test(f2, td, [&]() { return sqrt(f2) * nrel < tol; });
+  };
+  int info = 1;
+  bool done = converged();
+  if (done) info = 0;
+  for (int inew = 1; !done && inew < P.newton_max_iter; ++inew) {
+    ac_jacobians_fp64(pt, lp.mu, rho, A, B);
     const double* W = lp.W;
     double M[9];  // -(A W + B)
 #pragma unroll
@@ -682,58 +771,54 @@ __device__ inline int nsn_newton_std_fp64(const LocalProblem<double>& lp, double
     }
     dR[0] = F[0]; dR[1] = F[1]; dR[2] = F[2];
     const int info3 = solve_3x3_gepp_select(M, dR);
-    if (info3) {
-      dR[0] = 0.0; dR[1] = 0.0; dR[2] = 0.0;
-    }
-    if (damped) {
-      if (!info3) {
-        double alpha = 1.0;
-        const double inf = 1e20;
-        double amin = 0.0, amax = inf;
-        const double q0 = 0.5 * *F2;
-        double dqdt0 = 0.0;
+    dR[0] = info3 ? 0.0 : dR[0];
+    dR[1] = info3 ? 0.0 : dR[1];
+    dR[2] = info3 ? 0.0 : dR[2];
+    // the step with t = 1: the undamped one, and the line search's first trial
+    const double q0 = 0.5 * f2;
+    double dqdt0 = 0.0;
 #pragma unroll
-        for (int i = 0; i < 3; i++)
-          dqdt0 += F[i] * -(M[i] * dR[0] + M[i + 3] * dR[1] + M[i + 6] * dR[2]);
-        for (int it = 0; it < P.ls_max_iter; it++) {
-          double rt[3];
-          AcStdPoint<double> unused;
+    for (int i = 0; i < 3; i++)
+      dqdt0 += F[i] * -(M[i] * dR[0] + M[i + 3] * dR[1] + M[i + 6] * dR[2]);
+    double rt[3] = {r[0] + dR[0], r[1] + dR[1], r[2] + dR[2]};
+    local_velocity<double>(lp, rt, v);
+    ac_point_fp64(rt, v, lp.mu, rho, F, pt);
+    f2 = F[0] * F[0] + F[1] * F[1] + F[2] * F[2];
+    if (damped && !info3) {
+      double alpha = 1.0, slope = 0.5 * f2 - q0, amin = 0.0, amax = 1e20;
+      int it = 0;
+      for (;;) {
+        const bool C1 = slope >= 0.9 * dqdt0, C2 = slope <= 0.1 * dqdt0;
+        if ((C1 && C2) || P.ls_max_iter <= 0) break;
+        if (!C1)
+          amin = alpha;
+        else
+          amax = alpha;
+        if (alpha < 1e20)
+          alpha = 0.5 * (amin + amax);
+        else
+          alpha = 10.0 * alpha;
 #pragma unroll
-          for (int i = 0; i < 3; i++) rt[i] = r[i] + alpha * dR[i];
-          local_velocity_inline<double>(lp, rt, v);
-          ac_std_f<double>(rt, v, lp.mu, rho, F, unused);
-          const double q = 0.5 * (F[0] * F[0] + F[1] * F[1] + F[2] * F[2]);
-          const double slope = (q - q0) / alpha;
-          const bool C1 = slope >= 0.9 * dqdt0;
-          const bool C2 = slope <= 0.1 * dqdt0;
-          if (C1 && C2) break;
-          if (!C1)
-            amin = alpha;
-          else
-            amax = alpha;
-          if (alpha < inf)
-            alpha = 0.5 * (amin + amax);
-          else
-            alpha = 10.0 * alpha;
-        }
-        t = alpha;
+        for (int i = 0; i < 3; i++) rt[i] = r[i] + alpha * dR[i];
+        local_velocity<double>(lp, rt, v);
+        ac_point_fp64(rt, v, lp.mu, rho, F, pt);
+        f2 = F[0] * F[0] + F[1] * F[1] + F[2] * F[2];
+        if (++it >= P.ls_max_iter) break;
+        slope = (0.5 * f2 - q0) / alpha;
       }
-      r[0] = r[0] + t * dR[0];
-      r[1] = r[1] + t * dR[1];
-      r[2] = r[2] + t * dR[2];
-    } else {
-      r[0] += dR[0]; r[1] += dR[1]; r[2] += dR[2];
     }
-    local_velocity<double>(lp, r, v);
-    ac_std_f<double>(r, v, lp.mu, rho, F, pt);
-    *F2 = F[0] * F[0] + F[1] * F[1] + F[2] * F[2];
+    r[0] = rt[0]; r[1] = rt[1]; r[2] = rt[2];
     if (damped && info3) break;
-    if (root_below(*F2, nrel, tol)) return 0;
-    if (root_below(dR[0] * dR[0] + dR[1] * dR[1] + dR[2] * dR[2], 1.0, 10.0 * DBL_EPSILON))
-      return 1;
-    if (info3) break;
+    if (converged()) {
+      info = 0;
+      break;
+    }
+    const double d2 = dR[0] * dR[0] + dR[1] * dR[1] + dR[2] * dR[2];
+    done = root_test(d2, 10.0 * DBL_EPSILON,
+                     [&]() { return sqrt(d2) < 10.0 * DBL_EPSILON; }) || info3;
   }
-  return 1;
+  *F2 = f2;
+  return info;
 }
 
 // onecontact...c:429-559 (damped = false) and 710-854 (damped = true)
@@ -926,15 +1011,26 @@ __device__ int hybrid_solve(const LocalProblem<T>& lp, T* r, const LocalParams& 
   T res = T(0), cur;
   if constexpr (sizeof(T) == 8) {
     // the starting error matters only where the Newton solution is not
-    // accepted by its own error, so it is evaluated only there
+    // accepted by its own error, so it is evaluated only there; the caller
+    // reads an accepted error only as a number not above 1 (the filter), which
+    // tol <= 1 bounds, so its root is taken only for a larger tol
     if (P.hybrid_strategy == 2) {
       info = hybrid_newton<T>(lp, r, P, tol, rho, &res);
-      const T e = compute_local_error<T>(lp, r);
+      const T nq = sqrt(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
+      T v[3];
+      local_velocity<T>(lp, r, v);
+      const T ue = unitary_error<T>(r, v, lp.mu);
+      auto error = [&]() {
+        const T x = sqrt(ue);
+        return nq > num<T>::eps ? x / nq : x;
+      };
       const bool number = !(isnan(res) || isinf(res));
-      if (number && e <= tol) {
-        *residual = e;
+      if (number && root_test(ue, nq > num<T>::eps ? tol * nq : tol,
+                              [&]() { return error() <= tol; })) {
+        *residual = tol <= T(1) ? tol : error();
         return info;
       }
+      const T e = error();
       cur = compute_local_error<T>(lp, bak);
       if (number && e <= cur) {
         cur = e;

@@ -82,7 +82,9 @@ __global__ __launch_bounds__(256, MINW) void k_sweep(SweepPtrs<T> P,
   if (P.fcnt) count_frozen(P, s, lane, len);
   light = wave_sum(light);
   nr2 = wave_sum(nr2);
-  if (lane == 0) {
+  if (P.part_rows) {
+    if (lane < 8) P.part[8 * (size_t)s + lane] = lane == 0 ? light : lane == 1 ? nr2 : 0.0;
+  } else if (lane == 0) {
     P.part[2 * (size_t)s] = light;
     P.part[2 * (size_t)s + 1] = nr2;
   }
@@ -128,6 +130,136 @@ __global__ __launch_bounds__(256, 2) void k_sweep_w4(SweepPtrs<T> P,
   if (lane == 0) {
     P.part[2 * (size_t)s] = light;
     P.part[2 * (size_t)s + 1] = nr2;
+  }
+}
+
+// One colour of one FP64 sweep with a workgroup of four waves per row of 16
+// contacts: lane 16 p + c of wave w gathers block 4 w + p (+ 16, + 32, ...) of
+// contact c, so a row's blocks and neighbour reactions are all loaded in two
+// memory round trips (columns, reactions) instead of two per four or eight
+// blocks; the products go through LDS and 48 lanes of wave 0 add them, one
+// component of one contact a lane, in the reference's row order
+// (mvp3x3: block after block, column after column), so the sums have the
+// same bits.  Wave 0 then solves the row's contacts.  A colour of a mid-sized
+// problem has far fewer slices than the GPU has SIMDs and its time is the
+// chain of one wave: 4 x the workgroups, each with a quarter of a slice's
+// address work, shorten it (50k random pairs, 23-104 slices a colour: 19.0 ->
+// 13.0 us a launch; 1000 contacts, 1-3 slices: 11.9 -> 9.9).  The arguments
+// that the first loads need come first, so that they arrive preloaded in
+// registers, and the slot's own loads follow the gather's.
+constexpr int ORD_PLANES = 32;  // planes per pass through LDS (36 KB)
+// A colour of more slices runs the one-wave kernel: with up to a slice a CU
+// the four workgroups of every slice are resident at once (two waves a SIMD).
+// A sweep of the 300k pile (colours of 877 down to 1 slices), us: limit 32,
+// 322; 128, 311; 192, 303; 256, 303; 400, 302; none, 375; all one-wave, 351.
+// The 1M pile: 256, 582; 500, 582; all one-wave, 599.
+constexpr int ORD_MAX_SLICES = 256;
+__global__ __launch_bounds__(256, 2) void k_sweep_ordered(const SolveState* __restrict__ st,
+                                                          const int2* __restrict__ planes,
+                                                          int s_begin, int s_end,
+                                                          const int* __restrict__ cols,
+                                                          const double* __restrict__ vals,
+                                                          const double4* reactions,
+                                                          const int* __restrict__ lens,
+                                                          const DevParams* __restrict__ prm,
+                                                          SweepPtrs<double> P) {
+  __shared__ double prod[ORD_PLANES * 9 * 16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int g = __builtin_amdgcn_readfirstlane(xcd_block(4 * (s_end - s_begin)));
+  const int s = s_begin + (g >> 2), row = g & 3;
+  if (s >= s_end) return;
+  const int c = lane & 15, p = wave * 4 + (lane >> 4);
+  const int sl = row * 16 + c;  // lane of the slice
+  const int stop = st->stop, phase = st->phase;
+  const int2 pl = planes[s];
+  const int koff = __builtin_amdgcn_readfirstlane(pl.x);
+  const int kmax = __builtin_amdgcn_readfirstlane(pl.y);
+  const StepConsts sc = step_consts<double>(prm);
+  const double tol = st->local_tol;
+  // wave 0: lanes 0-15 the contacts' local problems, lanes 0-47 their q
+  SlotInputs<double> in;
+  double y = 0.0;
+  const int comp = lane >> 4;
+  int len = -1;
+  const int* __restrict__ colp = cols + (size_t)koff * 64 + sl;
+  const double* __restrict__ valp = vals + (size_t)koff * 9 * 64 + sl;
+  double rho[3] = {0.0, 0.0, 0.0};
+  for (int k0 = 0;; k0 += ORD_PLANES) {
+    constexpr int U = ORD_PLANES / 16;
+    int j[U];
+    double w[U][9];
+    double4 rj[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = k0 + p + 16 * u;
+      if (k < kmax) {
+        j[u] = colp[(size_t)k * 64];
+#pragma unroll
+        for (int e = 0; e < 9; e++) w[u][e] = valp[((size_t)k * 9 + e) * 64];
+      }
+    }
+    if (k0 == 0) {
+      // after the gather's first loads, which the slot's then do not delay
+      len = lens[s * 64 + sl];
+      if (wave == 0) {
+        if (comp < 3) y = P.q[(size_t)(s * 3 + comp) * 64 + sl];
+        if (comp == 0) load_slot<double>(P, s, sl, &in);
+      }
+      step_consts_ready(sc);
+      asm volatile("" ::"s"(tol), "s"(stop), "s"(phase));
+      if (stop || phase != 0) return;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (k0 + p + 16 * u < kmax) rj[u] = reactions[j[u]];
+    if (wave == 0 && comp == 0 && k0 == 0)
+      compute_rho<double>(sc.rho_strategy, sc.rho_constant, in.lp.W, rho);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k0 + p + 16 * u < kmax) {
+        double* o = prod + (size_t)((p + 16 * u) * 9) * 16 + c;
+        // a padded block is zero and reads the slot's own reaction: its
+        // products are made zeros here, so the sum needs no test
+        const bool live = k0 + p + 16 * u < len;
+        const double v[3] = {live ? rj[u].x : 0.0, live ? rj[u].y : 0.0, live ? rj[u].z : 0.0};
+#pragma unroll
+        for (int e = 0; e < 9; e++) o[e * 16] = w[u][e] * v[e / 3];
+      }
+    }
+    __syncthreads();
+    if (wave == 0 && comp < 3) {
+      const int n = min(kmax - k0, ORD_PLANES);
+      const double* a = prod + comp * 16 + c;
+      int k = 0;
+      for (; k + 4 <= n; k += 4) {
+        double t[12];
+#pragma unroll
+        for (int e = 0; e < 12; e++) t[e] = a[(k * 9 + 3 * e) * 16];
+#pragma unroll
+        for (int e = 0; e < 12; e++) y += t[e];
+      }
+      for (; k < n; k++) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) y += a[(k * 9 + 3 * e) * 16];
+      }
+    }
+    if (k0 + ORD_PLANES >= kmax) break;
+    __syncthreads();
+  }
+  if (wave != 0) return;
+  const double y1 = __shfl(y, c + 16, 64), y2 = __shfl(y, c + 32, 64);
+  double light = 0.0, nr2 = 0.0;
+  if (comp == 0 && len >= 0) {
+    in.ql[0] = y;
+    in.ql[1] = y1;
+    in.ql[2] = y2;
+    finish_slot<double>(P, sc, s, sl, tol, in, &light, &nr2, nullptr, rho);
+  }
+  light = row_sum(light);
+  nr2 = row_sum(nr2);
+  if (lane == 0) {
+    P.part[2 * (size_t)(4 * s + row)] = light;
+    P.part[2 * (size_t)(4 * s + row) + 1] = nr2;
   }
 }
 
@@ -275,12 +407,16 @@ __global__ __launch_bounds__(256) void k_residual(SweepPtrs<double> P, const Sol
 // sweep (fc3d_nsgs.c:726-735).
 __global__ __launch_bounds__(1024) void k_finalize_sweep(const DevParams* prm, SolveState* st,
                                                          const double* part, int nslices,
-                                                         int want_phase, const int* fcnt) {
+                                                         int want_phase, const int* fcnt,
+                                                         int rows) {
   __shared__ double sh[2 * 16];
   __shared__ int nfrozen;
   if (st->stop || st->phase != want_phase) return;
   double sums[2];
-  block_sums<2>(part, nslices, sh, sums);
+  if (rows)  // k_sweep_ordered's partials
+    block_sums<2, 1024, true>(part, nslices, sh, sums);
+  else
+    block_sums<2>(part, nslices, sh, sums);
   if (fcnt) {
     if (threadIdx.x == 0) nfrozen = 0;
     __syncthreads();
@@ -503,6 +639,7 @@ struct fc3d_hip_problem {
   std::vector<int> colour;            // per original contact
   std::vector<int> colour_slice_ptr;  // ncolours + 1
   int* d_cps = nullptr;               // the same on the device
+  int2* d_planes = nullptr;           // per slice: koff and kmax together
   std::vector<int> slot2orig;         // -1 for padding
   std::vector<int> orig2slot;
   std::vector<double> colour_bytes64, colour_bytes32;  // algorithmic bytes per colour pass
@@ -799,14 +936,14 @@ static int ensure_fp32(fc3d_hip_problem* h) {
 static const char* const kScheduleNames[FC3D_NUM_SCHEDULES + 1] = {
     "auto", "u4/u8 occ2", "u4/u8 occ3", "u4/u8 occ4", "u4/u8 pf16 occ2", "u4/u8 pf16 occ3",
     "u2/u4 pf8 occ4", "single launch, u4/u8 occ2", "u8/u16 occ1", "u8/u16 pf16 occ1",
-    "fp32: four waves per slice, u4"};
+    "fp32: four waves per slice, u4; fp64: four waves per row of 16, ordered"};
 
 // With events, the launch goes through hipExtLaunchKernelGGL, which stamps
 // them with the dispatch's own start and end (the times a kernel-trace
 // profiler reports) instead of enqueuing separate marker packets.
 template <int U64, int U32, int PF, int MINW>
 static void launch_sweep_t(fc3d_hip_problem* h, int phase, int grid, int sb, int se,
-                           hipEvent_t e0, hipEvent_t e1) {
+                           hipEvent_t e0, hipEvent_t e1, int rows = 0) {
   if (phase) {
     auto k = k_sweep<float, U32, PF, MINW>;
     SweepPtrs<float> P = ptrs32(h);
@@ -819,6 +956,7 @@ static void launch_sweep_t(fc3d_hip_problem* h, int phase, int grid, int sb, int
   } else {
     auto k = k_sweep<double, U64, PF, MINW>;
     SweepPtrs<double> P = ptrs64(h, h->part);
+    P.part_rows = rows;
     if (h->accel_on) P.f = h->aa64.f;
     if (e0)
       hipExtLaunchKernelGGL(k, dim3(grid), dim3(256), 0, h->stream, e0, e1, 0, P, h->prm,
@@ -840,8 +978,37 @@ static void launch_sweep_w4(fc3d_hip_problem* h, int sb, int se, hipEvent_t e0, 
     hipLaunchKernelGGL(k, g, b, 0, h->stream, P, h->prm, h->st, sb, se, 1);
 }
 
+// Whether the sweep of this phase runs k_sweep_ordered: schedule 10 in FP64.
+// Contact freezing counts a slice's frozen contacts in one wave, which the
+// ordered kernel's four workgroups a slice do not do; it takes the one-wave
+// kernel instead (the same bits).
+static bool ordered_sweep(const fc3d_hip_problem* h, int phase, int schedule) {
+  return schedule == FC3D_SCHEDULE_W4 && !phase && !h->vel_on && h->freeze == 0;
+}
+
+static void launch_sweep_ordered(fc3d_hip_problem* h, int sb, int se, hipEvent_t e0,
+                                 hipEvent_t e1) {
+  SweepPtrs<double> P = ptrs64(h, h->part);
+  if (h->accel_on) P.f = h->aa64.f;
+  const dim3 g((unsigned)(4 * (se - sb))), b(256);
+  if (e0)
+    hipExtLaunchKernelGGL(k_sweep_ordered, g, b, 0, h->stream, e0, e1, 0,
+                          (const SolveState*)h->st, (const int2*)h->d_planes, sb, se, P.col, P.vals,
+                          (const double4*)P.r, P.len, (const DevParams*)h->prm, P);
+  else
+    hipLaunchKernelGGL(k_sweep_ordered, g, b, 0, h->stream, h->st, h->d_planes, sb, se, P.col,
+                       P.vals, P.r, P.len, h->prm, P);
+}
+
 static void launch_sweep(fc3d_hip_problem* h, int phase, int schedule, int grid, int sb, int se,
                          hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
+  if (ordered_sweep(h, phase, schedule)) {
+    if (se - sb <= ORD_MAX_SLICES)
+      launch_sweep_ordered(h, sb, se, e0, e1);
+    else
+      launch_sweep_t<8, 16, 0, 1>(h, phase, grid, sb, se, e0, e1, 1);
+    return;
+  }
   if (schedule == FC3D_SCHEDULE_W4 && phase) {
     launch_sweep_w4(h, sb, se, e0, e1);
     return;
@@ -1039,7 +1206,8 @@ static void enqueue_sweep(fc3d_hip_problem* h, int phase, int schedule, hipEvent
   if (!h->vel_on || vel_tail_begin(h, phase) >= h->ncolours)
     hipLaunchKernelGGL(k_finalize_sweep, dim3(1), dim3(1024), 0, h->stream, h->prm, h->st,
                        h->part, h->nslices, phase,
-                       (const int*)(h->freeze > 0 && !phase ? h->d_fcnt : nullptr));
+                       (const int*)(h->freeze > 0 && !phase ? h->d_fcnt : nullptr),
+                       ordered_sweep(h, phase, schedule) ? 1 : 0);
   if (!phase) {
     hipLaunchKernelGGL(k_residual, dim3((h->nslices + 3) / 4), dim3(256), 0, h->stream,
                        ptrs64(h, h->part2), h->st, h->nslices, 0, nullptr, 0);
@@ -1639,14 +1807,16 @@ int fc3d_hip_problem_create(int nc, const int64_t* row_ptr, const int64_t* col_i
   h->colour_nc.assign(h->colour_slice_ptr.size() - 1, 0.0);
   for (int c : h->colour) h->colour_nc[(size_t)c] += 1.0;
   build_dataflow(L, h->colour.data(), &h->dfh);
-  if ((rc = dev_upload(&h->len, L.len)) || (rc = dev_upload(&h->dpos, L.dpos)) ||
+  std::vector<int2> planes((size_t)L.nslices);
+  for (size_t k = 0; k < planes.size(); k++) planes[k] = make_int2(L.koff[k], L.kmax[k]);
+  if ((rc = dev_upload(&h->d_planes, planes)) || (rc = dev_upload(&h->len, L.len)) || (rc = dev_upload(&h->dpos, L.dpos)) ||
       (rc = dev_upload(&h->koff, L.koff)) || (rc = dev_upload(&h->kmax, L.kmax)) ||
       (rc = dev_upload(&h->col, L.col)) || (rc = dev_upload(&h->vals, L.vals)) ||
       (rc = dev_upload(&h->diag, L.diag)) || (rc = dev_upload(&h->q, L.q)) ||
       (rc = dev_upload(&h->mu, L.mu)) || (rc = dev_alloc(&h->r, (size_t)h->nslots)) ||
       (rc = dev_alloc(&h->u, (size_t)h->nslots)) || (rc = dev_alloc(&h->x, (size_t)h->nslots)) ||
       (rc = dev_alloc(&h->pli, (size_t)h->nslots)) ||
-      (rc = dev_alloc(&h->part, 2 * (size_t)h->nslices)) ||
+      (rc = dev_alloc(&h->part, 8 * (size_t)h->nslices)) ||
       (rc = dev_alloc(&h->part2, 3 * (size_t)h->nslices)) || (rc = dev_alloc(&h->prm, 1)) ||
       (rc = dev_alloc(&h->st, 1)))
     return fail(rc);
@@ -1674,7 +1844,7 @@ void fc3d_hip_problem_destroy(fc3d_hip_problem* h) {
   free_accel(h);
   free_stage_bufs(h);
   void* dfp[] = {h->dep_ptr, h->dep_idx, h->qlist, h->done,    h->df,    h->d_block_dst,
-                 h->d_o2s,    h->d_cps,    h->d_ba,   h->d_bb,   h->d_inc_ptr, h->d_inc, h->d_H,
+                 h->d_o2s,    h->d_cps,    h->d_planes,   h->d_ba,   h->d_bb,   h->d_inc_ptr, h->d_inc, h->d_H,
                  h->d_minv,   h->d_vfree,  h->d_V,    h->d_H32,     h->d_minv32, h->d_V32,
                  h->d_F,      h->d_F32,    h->d_frz,  h->d_le2,  h->d_fcnt,
                  h->d_fs,     h->d_bmark,  h->d_slice_colour, h->d_focus_cnt,

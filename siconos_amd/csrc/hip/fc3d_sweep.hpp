@@ -74,6 +74,7 @@ struct SweepPtrs {
   T* pli;           // per-slot PLI step (persistent local state); null when the
                     // local solver keeps none (550, 551, 552): not loaded, not stored
   double* part;     // per-slice partial sums
+  int part_rows = 0;  // 1: four entries a slice (block_sums' ROWS), the sums in the first
   typename vec4<T>::type* f = nullptr;  // if set: r_new - r_old of the sweep
   // contact freezing (FP64 sweeps; null when off): per-slot counters of the
   // sweeps still to skip, the slot's last light-error term, per-slice counts
@@ -119,11 +120,17 @@ __device__ __forceinline__ double swap_add(double v) {
 // steps each quad holds one value, so the half-row mirror (lane 7 - i of each
 // 8) reads what lane ^ 4 holds, and likewise the row mirror for ^ 8; the
 // permlane swaps for ^ 16 and ^ 32.  Call with every lane active.
-__device__ __forceinline__ double wave_sum(double v) {
+// wave_sum's first four steps: the sum over each row of 16 lanes.
+__device__ __forceinline__ double row_sum(double v) {
   v = dpp_add<0xB1>(v);   // quad_perm [1,0,3,2]
   v = dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
   v = dpp_add<0x141>(v);  // row_half_mirror
   v = dpp_add<0x140>(v);  // row_mirror
+  return v;
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+  v = row_sum(v);
   v = swap_add<16>(v);
   v = swap_add<32>(v);
   return v;
@@ -136,9 +143,19 @@ __device__ __forceinline__ double wave_sum(double v) {
 // wave_sum, then the 16 wave sums are added in order.  A workgroup of R
 // threads (R divides 1024, R >= 64) computes the same bits: thread r stands
 // for threads r, r + R, ..., and its wave for the matching waves.  sh holds
-// NV * 16 doubles; the results are valid on thread 0.
-template <int NV, int R = 1024>
+// NV * 16 doubles; the results are valid on thread 0.  ROWS: part holds four
+// entries per slice, the row_sums of its 16-lane rows, added here as wave_sum
+// adds them ((row 0 + row 1) + (row 2 + row 3)).
+template <int NV, int R = 1024, bool ROWS = false>
 __device__ void block_sums(const double* __restrict__ part, int n, double* sh, double* out) {
+  auto entry = [&](int k, int j) {
+    if constexpr (ROWS) {
+      const double* p = part + (size_t)k * 4 * NV + j;
+      return (p[0] + p[NV]) + (p[2 * NV] + p[3 * NV]);
+    } else {
+      return part[(size_t)k * NV + j];
+    }
+  };
   static_assert(R >= 64 && R <= 1024 && 1024 % R == 0, "R must divide 1024");
   constexpr int M = 1024 / R;          // threads each real thread stands for
   constexpr int MB = M < 2 ? M : 2;    // of those, loaded together
@@ -159,7 +176,7 @@ __device__ void block_sums(const double* __restrict__ part, int n, double* sh, d
         for (int u = 0; u < 16; u++) {
           const int k = base + (int)threadIdx.x + (m0 + mm) * R + u * 1024;
 #pragma unroll
-          for (int j = 0; j < NV; j++) t[mm][u][j] = k < n ? part[(size_t)k * NV + j] : 0.0;
+          for (int j = 0; j < NV; j++) t[mm][u][j] = k < n ? entry(k, j) : 0.0;
         }
 #pragma unroll
       for (int mm = 0; mm < MB; mm++)
@@ -307,11 +324,14 @@ __device__ __forceinline__ void gather_row(const SweepPtrs<T>& P, int s, int lan
 // Workgroups are dispatched round-robin over the 8 XCDs (block b on XCD
 // b % 8).  This maps the blocks of each XCD onto one contiguous range of
 // slices, so that the neighbour gathers of an XCD stay within its own L2.
-__device__ __forceinline__ int xcd_block() {
-  const int b = blockIdx.x, nb = gridDim.x;
+// nb: the grid's size (a caller that knows it from an argument spares the
+// load of the launch's dimensions).
+__device__ __forceinline__ int xcd_block(int nb) {
+  const int b = blockIdx.x;
   const int x = b & 7, q = nb >> 3, rem = nb & 7;
   return x * q + (x < rem ? x : rem) + (b >> 3);
 }
+__device__ __forceinline__ int xcd_block() { return xcd_block((int)gridDim.x); }
 
 // Inputs of one slot's local solve: diagonal block, mu, the old reaction and
 // the persistent PLI step; q_loc starts at the slot's q.
@@ -389,14 +409,54 @@ __device__ __forceinline__ void step_consts_ready(const StepConsts& c) {
                "s"(c.rho_constant), "s"(c.omega));
 }
 
-// Local solve, relaxation, light-error term, optional filter and write-back
-// for a slot whose local q (q + sum_j W_ij r_j) is in in->ql.
+// Local solve, relaxation, light-error term and optional filter of a slot
+// whose local q (q + sum_j W_ij r_j) is in in->ql: the accepted reaction in
+// out, the PLI step in in->pli, |r_old - r_new|^2 in *light (r_new in lr).
+// rho_in: the slot's AC parameters if the caller has them already.
+template <typename T>
+__device__ __forceinline__ void solve_slot(const StepConsts& c, T tol, SlotInputs<T>& in,
+                                           const T* rho_in, T* lr, double* light,
+                                           typename vec4<T>::type* out) {
+  LocalProblem<T>& lp = in.lp;
+  const typename vec4<T>::type ro = in.ro;
+  lp.q[0] = in.ql[0]; lp.q[1] = in.ql[1]; lp.q[2] = in.ql[2];
+  const T rold[3] = {ro.x, ro.y, ro.z};
+  lr[0] = ro.x; lr[1] = ro.y; lr[2] = ro.z;
+  T rho[3];
+  if (rho_in) {
+    rho[0] = rho_in[0]; rho[1] = rho_in[1]; rho[2] = rho_in[2];
+  } else {
+    compute_rho<T>(c.rho_strategy, T(c.rho_constant), lp.W, rho);
+  }
+  T res = T(0);
+  local_solve<T>(lp, lr, c.lp, tol, &in.pli, rho, &res);
+  if (c.relaxation) {
+    const T om = T(c.omega);
+#pragma unroll
+    for (int e = 0; e < 3; e++) lr[e] = om * lr[e] + (T(1) - om) * rold[e];
+  }
+  const T d0 = rold[0] - lr[0], d1 = rold[1] - lr[1], d2 = rold[2] - lr[2];
+  *light = double(d0 * d0 + d1 * d1 + d2 * d2);
+  const bool accept = !(c.filter && (isnan(res) || isinf(res) || res > T(1)));
+  *out = ro;
+  if (accept) { out->x = lr[0]; out->y = lr[1]; out->z = lr[2]; }
+}
+
+// The squared norm of an accepted reaction.
+template <typename T>
+__device__ __forceinline__ double squared_norm(const typename vec4<T>::type& out) {
+  return sizeof(T) == 8 ? double(out.x * out.x + out.y * out.y + out.z * out.z)
+                        : double(out.x) * double(out.x) + double(out.y) * double(out.y) +
+                              double(out.z) * double(out.z);
+}
+
+// solve_slot with contact freezing and the write-back to the slot.
 template <typename T>
 __device__ __forceinline__ void finish_slot(const SweepPtrs<T>& P, const StepConsts& c, int s,
                                             int lane, T tol, SlotInputs<T>& in, double* light,
-                                            double* nr2, typename vec4<T>::type* out_r = nullptr) {
+                                            double* nr2, typename vec4<T>::type* out_r = nullptr,
+                                            const T* rho_in = nullptr) {
   const int slot = s * 64 + lane;
-  LocalProblem<T>& lp = in.lp;
   const typename vec4<T>::type ro = in.ro;
   if (P.frz) {
     // fc3d_nsgs.c:749-756: a frozen contact keeps its reaction and adds its
@@ -410,21 +470,9 @@ __device__ __forceinline__ void finish_slot(const SweepPtrs<T>& P, const StepCon
       return;
     }
   }
-  T pli = in.pli;
-  lp.q[0] = in.ql[0]; lp.q[1] = in.ql[1]; lp.q[2] = in.ql[2];
-  const T rold[3] = {ro.x, ro.y, ro.z};
-  T lr[3] = {ro.x, ro.y, ro.z};
-  T rho[3];
-  compute_rho<T>(c.rho_strategy, T(c.rho_constant), lp.W, rho);
-  T res = T(0);
-  local_solve<T>(lp, lr, c.lp, tol, &pli, rho, &res);
-  if (c.relaxation) {
-    const T om = T(c.omega);
-#pragma unroll
-    for (int e = 0; e < 3; e++) lr[e] = om * lr[e] + (T(1) - om) * rold[e];
-  }
-  const T d0 = rold[0] - lr[0], d1 = rold[1] - lr[1], d2 = rold[2] - lr[2];
-  *light = double(d0 * d0 + d1 * d1 + d2 * d2);
+  T lr[3];
+  typename vec4<T>::type out;
+  solve_slot<T>(c, tol, in, rho_in, lr, light, &out);
   if (P.frz) {
     // fc3d_nsgs.c:723-724, 776-800: freeze the contact for P.freeze sweeps
     // when its step is small against its reaction, or its reaction small
@@ -438,20 +486,15 @@ __device__ __forceinline__ void finish_slot(const SweepPtrs<T>& P, const StepCon
     const bool relative = l2 <= crit1 * sq, small = sq <= crit2;
     P.frz[slot] = ((relative || small) && fs->iter + 1 >= 10) ? P.freeze : 0;
   }
-  const bool accept = !(c.filter && (isnan(res) || isinf(res) || res > T(1)));
-  typename vec4<T>::type out = ro;
-  if (accept) { out.x = lr[0]; out.y = lr[1]; out.z = lr[2]; }
   P.r[slot] = out;
-  if (P.pli) P.pli[slot] = pli;
+  if (P.pli) P.pli[slot] = in.pli;
   if (out_r) *out_r = out;
   if (P.f) {
     typename vec4<T>::type d = out;
     d.x -= ro.x; d.y -= ro.y; d.z -= ro.z; d.w = T(0);
     P.f[slot] = d;
   }
-  *nr2 = sizeof(T) == 8 ? double(out.x * out.x + out.y * out.y + out.z * out.z)
-                        : double(out.x) * double(out.x) + double(out.y) * double(out.y) +
-                              double(out.z) * double(out.z);
+  *nr2 = squared_norm<T>(out);
 }
 
 template <typename T>

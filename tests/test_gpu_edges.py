@@ -155,3 +155,20 @@ def test_the_edge_cases_in_one_batch(oracle, star, schedule):
         np.testing.assert_array_equal(u[3 * c0:3 * (c0 + W.nc)], uo, err_msg=f"problem {k}")
         np.testing.assert_allclose(res[k], reso, rtol=1e-12)
     assert s.converged == len(probs)
+
+
+@pytest.mark.parametrize("kind", ["star", "wide"])
+def test_ordered_sweep_edges(oracle, star, kind):
+    """Schedule 10 on rows longer than one pass of its gather (99 blocks), and
+    on one colour of more slices than its own kernel takes, with rows of no
+    off-diagonal block and a ragged last slice."""
+    if kind == "star":
+        n, ba, bb, W, q, H, minv, vfree, mu = star
+        plain_matches_oracle(oracle, W, q, mu, tol=1e-8, schedule=10)
+        return
+    nc = 64 * 256 + 65
+    rng = np.random.default_rng(5)
+    M = rng.normal(size=(nc, 3, 3))
+    W = N.SparseBlock3(np.arange(nc + 1), np.arange(nc), M @ M.transpose(0, 2, 1) + np.eye(3))
+    plain_matches_oracle(oracle, W, rng.normal(size=3 * nc), rng.uniform(0.1, 0.9, nc), tol=1e-10,
+                         schedule=10)
