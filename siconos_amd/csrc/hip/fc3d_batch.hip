@@ -19,6 +19,7 @@
 #include "fc3d_internal.hpp"
 #include "fc3d_layout.hpp"
 #include "fc3d_sweep.hpp"
+#include "fc3d_transfer.hpp"
 
 namespace fc3d {
 
@@ -238,6 +239,7 @@ struct fc3d_hip_batch {
   float *vals32 = nullptr, *diag32 = nullptr, *q32 = nullptr, *mu32 = nullptr, *pli32 = nullptr;
   float4* r32 = nullptr;
   DevParams* prm = nullptr;
+  mutable Transfer transfer;  // reactions and velocities in the caller's order
   int tuned_wpp[2] = {0, 0};
 };
 
@@ -448,6 +450,7 @@ void fc3d_hip_batch_destroy(fc3d_hip_batch* b) {
                   b->vals32, b->diag32, b->q32,    b->mu32,    b->pli32,   b->r32,    b->prm};
   for (void* p : ptrs)
     if (p) hipFree(p);
+  b->transfer.release();
   if (b->stream) hipStreamDestroy(b->stream);
   delete b;
 }
@@ -463,25 +466,14 @@ int fc3d_hip_batch_order(const fc3d_hip_batch* b, int* order) {
 int fc3d_hip_batch_set_reaction(fc3d_hip_batch* b, const double* reaction) {
   if (!b || !reaction) return NUMERICS_ERR_NULL_POINTER;
   int rc = use_device(b->device);
-  if (rc) return rc;
-  std::vector<double4> buf((size_t)b->nslots, make_double4(0, 0, 0, 0));
-  for (int i = 0; i < b->ntotal; i++)
-    buf[(size_t)b->orig2slot[(size_t)i]] =
-        make_double4(reaction[3 * i], reaction[3 * i + 1], reaction[3 * i + 2], 0.0);
-  FC3D_HIP_TRY(hipMemcpy(b->r, buf.data(), sizeof(double4) * buf.size(), hipMemcpyHostToDevice));
-  return 0;
+  if (rc || (rc = b->transfer.ensure(b->orig2slot, b->slot2orig))) return rc;
+  return b->transfer.to_device(b->ntotal, b->nslots, reaction, b->r, b->stream);
 }
 
 static int batch_get(const fc3d_hip_batch* b, const double4* d, double* out) {
   int rc = use_device(b->device);
-  if (rc) return rc;
-  std::vector<double4> buf((size_t)b->nslots);
-  FC3D_HIP_TRY(hipMemcpy(buf.data(), d, sizeof(double4) * buf.size(), hipMemcpyDeviceToHost));
-  for (int i = 0; i < b->ntotal; i++) {
-    const double4 v = buf[(size_t)b->orig2slot[(size_t)i]];
-    out[3 * i] = v.x; out[3 * i + 1] = v.y; out[3 * i + 2] = v.z;
-  }
-  return 0;
+  if (rc || (rc = b->transfer.ensure(b->orig2slot, b->slot2orig))) return rc;
+  return b->transfer.to_host(b->ntotal, d, out, b->stream);
 }
 
 int fc3d_hip_batch_get_reaction(const fc3d_hip_batch* b, double* reaction) {

@@ -32,6 +32,7 @@
 #include "fc3d_layout.hpp"
 #include "fc3d_mlp.hpp"
 #include "fc3d_sweep.hpp"
+#include "fc3d_transfer.hpp"
 #include "fc3d_fp32_kernels.hpp"
 
 // instantiated in fc3d_fp32.hip (built with FMA contraction)
@@ -681,6 +682,7 @@ struct fc3d_hip_problem {
   int *dep_ptr = nullptr, *dep_idx = nullptr, *qlist = nullptr, *done = nullptr;
   DataflowState* df = nullptr;
   // in-place updates: CSR block -> layout position, uploaded on first use
+  mutable Transfer transfer;  // reactions and velocities in the caller's order
   std::vector<int64_t> block_dst;
   int64_t* d_block_dst = nullptr;
   int* d_o2s = nullptr;
@@ -1843,6 +1845,7 @@ void fc3d_hip_problem_destroy(fc3d_hip_problem* h) {
     if (p) hipFree(p);
   free_accel(h);
   free_stage_bufs(h);
+  h->transfer.release();
   void* dfp[] = {h->dep_ptr, h->dep_idx, h->qlist, h->done,    h->df,    h->d_block_dst,
                  h->d_o2s,    h->d_cps,    h->d_planes,   h->d_ba,   h->d_bb,   h->d_inc_ptr, h->d_inc, h->d_H,
                  h->d_minv,   h->d_vfree,  h->d_V,    h->d_H32,     h->d_minv32, h->d_V32,
@@ -1875,25 +1878,14 @@ int fc3d_hip_problem_order(const fc3d_hip_problem* h, int* order) {
 int fc3d_hip_set_reaction(fc3d_hip_problem* h, const double* reaction) {
   if (!h || !reaction) return NUMERICS_ERR_NULL_POINTER;
   int rc = use_device(h->device);
-  if (rc) return rc;
-  std::vector<double4> buf((size_t)h->nslots, make_double4(0, 0, 0, 0));
-  for (int i = 0; i < h->nc; i++)
-    buf[(size_t)h->orig2slot[(size_t)i]] =
-        make_double4(reaction[3 * i], reaction[3 * i + 1], reaction[3 * i + 2], 0.0);
-  FC3D_HIP_TRY(hipMemcpy(h->r, buf.data(), sizeof(double4) * buf.size(), hipMemcpyHostToDevice));
-  return 0;
+  if (rc || (rc = h->transfer.ensure(h->orig2slot, h->slot2orig))) return rc;
+  return h->transfer.to_device(h->nc, h->nslots, reaction, h->r, h->stream);
 }
 
 static int get_vec(const fc3d_hip_problem* h, const double4* d, double* out) {
   int rc = use_device(h->device);
-  if (rc) return rc;
-  std::vector<double4> buf((size_t)h->nslots);
-  FC3D_HIP_TRY(hipMemcpy(buf.data(), d, sizeof(double4) * buf.size(), hipMemcpyDeviceToHost));
-  for (int i = 0; i < h->nc; i++) {
-    const double4 v = buf[(size_t)h->orig2slot[(size_t)i]];
-    out[3 * i] = v.x; out[3 * i + 1] = v.y; out[3 * i + 2] = v.z;
-  }
-  return 0;
+  if (rc || (rc = h->transfer.ensure(h->orig2slot, h->slot2orig))) return rc;
+  return h->transfer.to_host(h->nc, d, out, h->stream);
 }
 
 int fc3d_hip_get_reaction(const fc3d_hip_problem* h, double* reaction) {

@@ -409,54 +409,16 @@ __device__ __forceinline__ void step_consts_ready(const StepConsts& c) {
                "s"(c.rho_constant), "s"(c.omega));
 }
 
-// Local solve, relaxation, light-error term and optional filter of a slot
-// whose local q (q + sum_j W_ij r_j) is in in->ql: the accepted reaction in
-// out, the PLI step in in->pli, |r_old - r_new|^2 in *light (r_new in lr).
-// rho_in: the slot's AC parameters if the caller has them already.
-template <typename T>
-__device__ __forceinline__ void solve_slot(const StepConsts& c, T tol, SlotInputs<T>& in,
-                                           const T* rho_in, T* lr, double* light,
-                                           typename vec4<T>::type* out) {
-  LocalProblem<T>& lp = in.lp;
-  const typename vec4<T>::type ro = in.ro;
-  lp.q[0] = in.ql[0]; lp.q[1] = in.ql[1]; lp.q[2] = in.ql[2];
-  const T rold[3] = {ro.x, ro.y, ro.z};
-  lr[0] = ro.x; lr[1] = ro.y; lr[2] = ro.z;
-  T rho[3];
-  if (rho_in) {
-    rho[0] = rho_in[0]; rho[1] = rho_in[1]; rho[2] = rho_in[2];
-  } else {
-    compute_rho<T>(c.rho_strategy, T(c.rho_constant), lp.W, rho);
-  }
-  T res = T(0);
-  local_solve<T>(lp, lr, c.lp, tol, &in.pli, rho, &res);
-  if (c.relaxation) {
-    const T om = T(c.omega);
-#pragma unroll
-    for (int e = 0; e < 3; e++) lr[e] = om * lr[e] + (T(1) - om) * rold[e];
-  }
-  const T d0 = rold[0] - lr[0], d1 = rold[1] - lr[1], d2 = rold[2] - lr[2];
-  *light = double(d0 * d0 + d1 * d1 + d2 * d2);
-  const bool accept = !(c.filter && (isnan(res) || isinf(res) || res > T(1)));
-  *out = ro;
-  if (accept) { out->x = lr[0]; out->y = lr[1]; out->z = lr[2]; }
-}
-
-// The squared norm of an accepted reaction.
-template <typename T>
-__device__ __forceinline__ double squared_norm(const typename vec4<T>::type& out) {
-  return sizeof(T) == 8 ? double(out.x * out.x + out.y * out.y + out.z * out.z)
-                        : double(out.x) * double(out.x) + double(out.y) * double(out.y) +
-                              double(out.z) * double(out.z);
-}
-
-// solve_slot with contact freezing and the write-back to the slot.
+// Local solve, relaxation, light-error term, optional filter and write-back
+// for a slot whose local q (q + sum_j W_ij r_j) is in in->ql.  rho_in: the
+// slot's AC parameters if the caller has them already.
 template <typename T>
 __device__ __forceinline__ void finish_slot(const SweepPtrs<T>& P, const StepConsts& c, int s,
                                             int lane, T tol, SlotInputs<T>& in, double* light,
                                             double* nr2, typename vec4<T>::type* out_r = nullptr,
                                             const T* rho_in = nullptr) {
   const int slot = s * 64 + lane;
+  LocalProblem<T>& lp = in.lp;
   const typename vec4<T>::type ro = in.ro;
   if (P.frz) {
     // fc3d_nsgs.c:749-756: a frozen contact keeps its reaction and adds its
@@ -470,9 +432,25 @@ __device__ __forceinline__ void finish_slot(const SweepPtrs<T>& P, const StepCon
       return;
     }
   }
-  T lr[3];
-  typename vec4<T>::type out;
-  solve_slot<T>(c, tol, in, rho_in, lr, light, &out);
+  T pli = in.pli;
+  lp.q[0] = in.ql[0]; lp.q[1] = in.ql[1]; lp.q[2] = in.ql[2];
+  const T rold[3] = {ro.x, ro.y, ro.z};
+  T lr[3] = {ro.x, ro.y, ro.z};
+  T rho[3];
+  if (rho_in) {
+    rho[0] = rho_in[0]; rho[1] = rho_in[1]; rho[2] = rho_in[2];
+  } else {
+    compute_rho<T>(c.rho_strategy, T(c.rho_constant), lp.W, rho);
+  }
+  T res = T(0);
+  local_solve<T>(lp, lr, c.lp, tol, &pli, rho, &res);
+  if (c.relaxation) {
+    const T om = T(c.omega);
+#pragma unroll
+    for (int e = 0; e < 3; e++) lr[e] = om * lr[e] + (T(1) - om) * rold[e];
+  }
+  const T d0 = rold[0] - lr[0], d1 = rold[1] - lr[1], d2 = rold[2] - lr[2];
+  *light = double(d0 * d0 + d1 * d1 + d2 * d2);
   if (P.frz) {
     // fc3d_nsgs.c:723-724, 776-800: freeze the contact for P.freeze sweeps
     // when its step is small against its reaction, or its reaction small
@@ -486,15 +464,20 @@ __device__ __forceinline__ void finish_slot(const SweepPtrs<T>& P, const StepCon
     const bool relative = l2 <= crit1 * sq, small = sq <= crit2;
     P.frz[slot] = ((relative || small) && fs->iter + 1 >= 10) ? P.freeze : 0;
   }
+  const bool accept = !(c.filter && (isnan(res) || isinf(res) || res > T(1)));
+  typename vec4<T>::type out = ro;
+  if (accept) { out.x = lr[0]; out.y = lr[1]; out.z = lr[2]; }
   P.r[slot] = out;
-  if (P.pli) P.pli[slot] = in.pli;
+  if (P.pli) P.pli[slot] = pli;
   if (out_r) *out_r = out;
   if (P.f) {
     typename vec4<T>::type d = out;
     d.x -= ro.x; d.y -= ro.y; d.z -= ro.z; d.w = T(0);
     P.f[slot] = d;
   }
-  *nr2 = squared_norm<T>(out);
+  *nr2 = sizeof(T) == 8 ? double(out.x * out.x + out.y * out.y + out.z * out.z)
+                        : double(out.x) * double(out.x) + double(out.y) * double(out.y) +
+                              double(out.z) * double(out.z);
 }
 
 template <typename T>

@@ -172,3 +172,18 @@ def test_ordered_sweep_edges(oracle, star, kind):
     W = N.SparseBlock3(np.arange(nc + 1), np.arange(nc), M @ M.transpose(0, 2, 1) + np.eye(3))
     plain_matches_oracle(oracle, W, rng.normal(size=3 * nc), rng.uniform(0.1, 0.9, nc), tol=1e-10,
                          schedule=10)
+
+
+@pytest.mark.parametrize("nc", [1, 63, 64, 65, 257, 3000])
+def test_reactions_come_back_in_the_callers_order(nc):
+    """set_reaction and reaction() at the edges of a slice and of a launch, for
+    a resident problem and for the same problem twice in a batch."""
+    g = N.generate_random_pairs(max(3, nc), nc, 0.2, 0.5, 9)
+    r = np.random.default_rng(nc).normal(size=3 * nc)
+    P = N.HipProblem(g.W, g.q, g.mu)
+    P.set_reaction(r)
+    np.testing.assert_array_equal(P.reaction(), r)
+    B = N.Batch([(g.W, g.q, g.mu)] * 2)
+    both = np.concatenate([r, -r])
+    B.set_reaction(both)
+    np.testing.assert_array_equal(B.reaction(), both)
