@@ -16,6 +16,7 @@
 #include <numeric>
 #include <vector>
 
+#include "fc3d_batch.hpp"
 #include "fc3d_internal.hpp"
 #include "fc3d_layout.hpp"
 #include "fc3d_sweep.hpp"
@@ -25,14 +26,6 @@ namespace fc3d {
 
 int colour_on_device(int nc, const int* d_rp, const int* d_ci, int* d_colour, hipStream_t s,
                      int* ncolours_out, std::vector<int>* host_colour);
-
-struct BatchProblem {
-  int cptr_off;     // first entry of the problem's colour slice pointers
-  int ncolours;
-  int slice_begin;
-  int slice_end;
-  double norm_q;
-};
 
 struct BatchArgs {
   SweepPtrs<double> P64;
@@ -46,6 +39,11 @@ struct BatchArgs {
   int* out_iter;
   int* out_fp32_iter;
   double* out_residual;
+  double* out_incr;  // last light error; may be null
+  // reactions in LDS: contacts numbered from 0 in slot order inside their
+  // problem (a colour's slices are full except its last)
+  const int* cbase;             // per slice: number of its first contact
+  const unsigned short* ccol;   // per plane entry: the neighbour's number
 };
 
 template <int WPP>
@@ -83,40 +81,227 @@ __device__ double problem_residual(const BatchArgs& A, const BatchProblem& d, do
   return err;
 }
 
+// One sweep of one problem with its reactions in LDS, by quads of four waves.
+// A quad takes a slice (up to 64 contacts of a colour; the problem's quads
+// take a colour's slices side by side): waves 0-2 each sum one component of
+// the slice's rows in the reference's order (mvp3x3), then wave 3 solves the
+// contacts, and while it does, waves 0-2 load the blocks of the quad's next
+// slice into registers (U planes of three values a lane), which no reaction
+// enters.  So a colour costs LDS gathers, two barriers and one wave's local
+// solves.  With each wave gathering and solving its own slice instead, the
+// dependent loads of W from L2 took as long as the solves (10 of 21 thousand
+// cycles a slice).
+// The two roles are loops of their own with the same barriers (each wave is in
+// one of them), so that their registers do not add up.
+struct QuadWalk {  // the quad's next slice; every quad walks the same steps
+  const int* cp;
+  int c, s0, se, s;
+  __device__ __forceinline__ QuadWalk(const int* cp_, int quad)
+      : cp(cp_), c(0), s0(cp_[0]), se(cp_[1]), s(cp_[0] + quad) {}
+  __device__ __forceinline__ bool active() const { return s < se; }
+  template <int NQ>
+  __device__ __forceinline__ bool next(int quad, int ncolours) {
+    s0 += NQ;
+    if (s0 >= se) {
+      if (++c >= ncolours) return false;
+      s0 = cp[c];
+      se = cp[c + 1];
+    }
+    s = s0 + quad;
+    return true;
+  }
+};
+
+template <typename T, int NQ, int U>
+__device__ __forceinline__ void quad_gather(const SweepPtrs<T>& P, const BatchArgs& A,
+                                            const BatchProblem& d,
+                                            const typename vec4<T>::type* r, T* q3, int role,
+                                            int quad, int lane) {
+  QuadWalk k(A.cptr + d.cptr_off, quad);
+  do {
+    if (k.active()) {
+      const int len = P.len[k.s * 64 + lane];
+      const int koff = __builtin_amdgcn_readfirstlane(P.koff[k.s]);
+      const int kmax = __builtin_amdgcn_readfirstlane(P.kmax[k.s]);
+      T acc = P.q[(size_t)(k.s * 3 + role) * 64 + lane];
+      const unsigned short* __restrict__ colp = A.ccol + (size_t)koff * 64;
+      const T* __restrict__ valp = P.vals + ((size_t)koff * 9 + role) * 64;
+      int jc[U];
+      T w[U][3];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (u < kmax) {
+          jc[u] = (colp + u * 64)[lane];
+#pragma unroll
+          for (int e = 0; e < 3; e++) w[u][e] = (valp + u * 576 + e * 192)[lane];
+        }
+      __syncthreads();  // the colours before have written their reactions
+      for (int k0 = 0;;) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (k0 + u < kmax) {
+            const typename vec4<T>::type rj = r[jc[u]];
+            T t = acc;
+            t += w[u][0] * rj.x;
+            t += w[u][1] * rj.y;
+            t += w[u][2] * rj.z;
+            acc = k0 + u < len ? t : acc;  // (a padded block is not added)
+            // four gathers in flight: all U at once would spill
+            if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+          }
+        k0 += U;
+        if (k0 >= kmax) break;
+        colp += U * 64;
+        valp += U * 576;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (k0 + u < kmax) {
+            jc[u] = (colp + u * 64)[lane];
+#pragma unroll
+            for (int e = 0; e < 3; e++) w[u][e] = (valp + u * 576 + e * 192)[lane];
+          }
+      }
+      q3[role * 64 + lane] = acc;
+    } else {
+      __syncthreads();
+    }
+    __syncthreads();  // the rows' sums
+  } while (k.next<NQ>(quad, d.ncolours));
+}
+
+template <typename T, int NQ>
+__device__ __forceinline__ void quad_solve(const SweepPtrs<T>& P, const BatchArgs& A,
+                                           const BatchProblem& d,
+                                           const DevParams* __restrict__ prm,
+                                           typename vec4<T>::type* r, const T* q3, T* pli, T tol,
+                                           int quad, int lane, double* light, double* nr2) {
+  const StepConsts sc = step_consts<T>(prm);
+  QuadWalk k(A.cptr + d.cptr_off, quad);
+  do {
+    if (k.active()) {
+      SlotInputs<T> in;
+      const int len = P.len[k.s * 64 + lane], id = A.cbase[k.s] + lane;
+#pragma unroll
+      for (int e = 0; e < 9; e++) in.lp.W[e] = P.diag[(size_t)(k.s * 9 + e) * 64 + lane];
+      in.lp.mu = P.mu[k.s * 64 + lane];
+      // (a padding lane's number may be the next slice's: not read)
+      in.pli = len >= 0 ? pli[id] : T(1);
+      T rho[3];
+      compute_rho<T>(sc.rho_strategy, T(sc.rho_constant), in.lp.W, rho);
+      __syncthreads();  // the gather reads the reactions
+      if (len >= 0) in.ro = r[id];
+      __syncthreads();  // the rows' sums
+      if (len >= 0) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) in.ql[e] = q3[e * 64 + lane];
+        SweepPtrs<T> Q;
+        Q.r = r;
+        Q.pli = pli;
+        Q.f = nullptr;
+        double l, n;
+        finish_slot<T>(Q, sc, id >> 6, id & 63, tol, in, &l, &n, nullptr, rho);
+        *light += l;
+        *nr2 += n;
+      }
+    } else {
+      __syncthreads();
+      __syncthreads();
+    }
+  } while (k.next<NQ>(quad, d.ncolours));
+}
+
+template <typename T, int NQ, int U>
+__device__ __forceinline__ void sweep_quads(const SweepPtrs<T>& P, const BatchArgs& A,
+                                            const BatchProblem& d,
+                                            const DevParams* __restrict__ prm,
+                                            typename vec4<T>::type* r, T* ql, T* pli, T tol,
+                                            int wave, int lane, double* light, double* nr2) {
+  // waves go to the CU's four SIMDs in turn: the quads' solving waves on
+  // different ones (76 -> 67 us a sweep of 500 contacts)
+  const int quad = wave >> 2, role = (wave + quad) & 3;
+  if (role < 3)
+    quad_gather<T, NQ, U>(P, A, d, r, ql + quad * 192, role, quad, lane);
+  else
+    quad_solve<T, NQ>(P, A, d, prm, r, ql + quad * 192, pli, tol, quad, lane, light, nr2);
+}
+
+// Copies a problem's reactions between its slots in HBM and LDS.
 template <int WPP>
-__global__ __launch_bounds__(64 * WPP, 2) void k_batch(BatchArgs A, const DevParams* __restrict__ prm,
-                                                    int mixed) {
+__device__ __forceinline__ void reactions_in(const BatchArgs& A, const BatchProblem& d,
+                                             double4* r) {
+  for (int slot = d.slice_begin * 64 + threadIdx.x; slot < d.slice_end * 64; slot += 64 * WPP)
+    if (A.P64.len[slot] >= 0) r[A.cbase[slot >> 6] + (slot & 63)] = A.P64.r[slot];
+}
+template <int WPP, typename T4>
+__device__ __forceinline__ void reactions_out(const BatchArgs& A, const BatchProblem& d,
+                                              const T4* r) {
+  for (int slot = d.slice_begin * 64 + threadIdx.x; slot < d.slice_end * 64; slot += 64 * WPP)
+    if (A.P64.len[slot] >= 0) {
+      const T4 x = r[A.cbase[slot >> 6] + (slot & 63)];
+      A.P64.r[slot] = make_double4(double(x.x), double(x.y), double(x.z), 0.0);
+    }
+}
+
+// LDS: the problem's reactions live in LDS (32 bytes a contact, FP64 or FP32)
+// and the sweeps run in quads of waves (sweep_quads); HBM holds the reactions
+// before, after, and for the residual.  A launch lasts as long as its slowest
+// problem, whose colours are one or two slices, so the chain of a colour is
+// what counts: 1024 problems of 8-512 contacts, at most 1000 sweeps, 139 -> 100
+// ms in FP64 and 63 -> 51 mixed; 64 problems 104 -> 83 and 54 -> 46.
+template <int WPP, bool LDS, bool MIXED>
+__global__ __launch_bounds__(64 * WPP, WPP == 8 ? 1 : 2) void k_batch(
+    BatchArgs A, const DevParams* __restrict__ prm) {
   __shared__ int sh_task;
   __shared__ double sh[WPP];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int NQ = WPP / 4;
+  __shared__ double ql[LDS ? NQ * 192 : 1];
+  extern __shared__ __align__(16) double4 r64[];
+  float4* const r32 = reinterpret_cast<float4*>(r64);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   for (;;) {
     if (threadIdx.x == 0) sh_task = atomicAdd(A.counter, 1);
     __syncthreads();
     const int t = sh_task;
     __syncthreads();
     if (t >= A.nprob) return;
-    const int p = A.order[t];
+    const int p = __builtin_amdgcn_readfirstlane(A.order[t]);
     const BatchProblem d = A.problems[p];
+    // (in LDS mode the PLI steps are kept by contact number)
+    double* const pli64 = A.P64.pli + d.slice_begin * 64;
+    float* const pli32 = A.P32.pli + d.slice_begin * 64;
     for (int slot = d.slice_begin * 64 + threadIdx.x; slot < d.slice_end * 64; slot += 64 * WPP) {
       A.P64.pli[slot] = 1.0;
-      if (mixed) {
+      if (MIXED) {
         const double4 x = A.P64.r[slot];
-        A.P32.r[slot] = make_float4(float(x.x), float(x.y), float(x.z), 0.f);
+        const float4 y = make_float4(float(x.x), float(x.y), float(x.z), 0.f);
+        if (!LDS)
+          A.P32.r[slot] = y;
+        else if (A.P64.len[slot] >= 0)
+          r32[A.cbase[slot >> 6] + (slot & 63)] = y;
         A.P32.pli[slot] = 1.0f;
       }
     }
+    if (LDS && !MIXED) reactions_in<WPP>(A, d, r64);
     __syncthreads();
-    int iter = 0, fp32_iter = 0, phase = mixed, notconv = 1;
+    int iter = 0, fp32_iter = 0, phase = MIXED ? 1 : 0, notconv = 1;
     double working_tol = prm->tol, local_tol = prm->local_tol, incr = INFINITY, full = INFINITY;
     int freq = prm->freq;
     const int mode = prm->mode;
     while (iter < prm->max_iter) {
       double light = 0.0, nr2 = 0.0;
+      if constexpr (LDS) {
+        if (MIXED && phase)
+          sweep_quads<float, NQ, 16>(A.P32, A, d, prm, r32, reinterpret_cast<float*>(ql), pli32,
+                                     float(prm->fp32_local_tol), wave, lane, &light, &nr2);
+        else
+          sweep_quads<double, NQ, 16>(A.P64, A, d, prm, r64, ql, pli64, local_tol, wave, lane,
+                                      &light, &nr2);
+      } else
       for (int c = 0; c < d.ncolours; c++) {
         const int sb = A.cptr[d.cptr_off + c], se = A.cptr[d.cptr_off + c + 1];
         for (int s = sb + wave; s < se; s += WPP) {
           double l, n;
-          if (phase)
+          if (MIXED && phase)
             sweep_slot<float, 8, 0>(A.P32, prm, s, lane, float(prm->fp32_local_tol), &l, &n);
           else
             sweep_slot<double, 4, 0>(A.P64, prm, s, lane, local_tol, &l, &n);
@@ -131,9 +316,17 @@ __global__ __launch_bounds__(64 * WPP, 2) void k_batch(BatchArgs A, const DevPar
       incr = sqrt(light);
       const double nr = sqrt(nr2);
       if (fabs(nr) > DBL_EPSILON) incr /= nr;
-      if (phase) {
+      if (MIXED && phase) {
         fp32_iter++;
-        if (incr < prm->fp32_tol || iter >= prm->max_iter) {
+        if (LDS && (incr < prm->fp32_tol || iter >= prm->max_iter)) {
+          reactions_out<WPP>(A, d, r32);
+          for (int id = threadIdx.x; id < (d.slice_end - d.slice_begin) * 64; id += 64 * WPP)
+            pli64[id] = double(pli32[id]);
+          __syncthreads();
+          reactions_in<WPP>(A, d, r64);
+          __syncthreads();
+          phase = 0;
+        } else if (incr < prm->fp32_tol || iter >= prm->max_iter) {
           for (int slot = d.slice_begin * 64 + threadIdx.x; slot < d.slice_end * 64;
                slot += 64 * WPP) {
             const float4 x = A.P32.r[slot];
@@ -151,6 +344,10 @@ __global__ __launch_bounds__(64 * WPP, 2) void k_batch(BatchArgs A, const DevPar
         if (incr >= working_tol) {
           notconv = 1;
         } else {
+          if (LDS) {
+            reactions_out<WPP>(A, d, r64);
+            __syncthreads();
+          }
           full = problem_residual<WPP>(A, d, sh);
           __syncthreads();
           const double user = prm->tol;
@@ -174,6 +371,10 @@ __global__ __launch_bounds__(64 * WPP, 2) void k_batch(BatchArgs A, const DevPar
       } else {
         const bool eval = freq > 0 ? (iter % freq == 0) : true;
         if (eval) {
+          if (LDS) {
+            reactions_out<WPP>(A, d, r64);
+            __syncthreads();
+          }
           full = problem_residual<WPP>(A, d, sh);
           __syncthreads();
           if (mode == SICONOS_NSGS_ERROR_EVALUATION_ADAPTIVE && freq > 0 && full > working_tol)
@@ -186,7 +387,13 @@ __global__ __launch_bounds__(64 * WPP, 2) void k_batch(BatchArgs A, const DevPar
       }
       if (!notconv) break;
     }
-    if (phase) {  // max_iter reached inside the FP32 phase: hand the iterate over
+    if (LDS) {
+      if (MIXED && phase)
+        reactions_out<WPP>(A, d, r32);
+      else
+        reactions_out<WPP>(A, d, r64);
+      __syncthreads();
+    } else if (MIXED && phase) {  // max_iter reached inside the FP32 phase: hand the iterate over
       for (int slot = d.slice_begin * 64 + threadIdx.x; slot < d.slice_end * 64;
            slot += 64 * WPP) {
         const float4 x = A.P32.r[slot];
@@ -205,6 +412,7 @@ __global__ __launch_bounds__(64 * WPP, 2) void k_batch(BatchArgs A, const DevPar
       A.out_iter[p] = iter;
       A.out_fp32_iter[p] = fp32_iter;
       A.out_residual[p] = full;
+      if (A.out_incr) A.out_incr[p] = incr;
     }
     __syncthreads();
   }
@@ -239,11 +447,34 @@ struct fc3d_hip_batch {
   float *vals32 = nullptr, *diag32 = nullptr, *q32 = nullptr, *mu32 = nullptr, *pli32 = nullptr;
   float4* r32 = nullptr;
   DevParams* prm = nullptr;
+  int *d_cbase = nullptr, max_nc = 0;
+  unsigned short* d_ccol = nullptr;
   mutable Transfer transfer;  // reactions and velocities in the caller's order
   int tuned_wpp[2] = {0, 0};
 };
 
 namespace fc3d {
+
+void number_contacts(const HostLayout& L, const std::vector<BatchProblem>& problems,
+                     std::vector<int>* cbase, std::vector<unsigned short>* ccol) {
+  cbase->assign((size_t)L.nslices, 0);
+  ccol->assign((size_t)L.nplanes * 64, 0);
+  for (const BatchProblem& d : problems) {
+    int n = 0;
+    for (int s = d.slice_begin; s < d.slice_end; s++) {
+      (*cbase)[(size_t)s] = n;
+      for (int l = 0; l < 64; l++) n += L.slot2orig[(size_t)s * 64 + (size_t)l] >= 0;
+    }
+    for (int s = d.slice_begin; s < d.slice_end; s++)
+      for (size_t e = (size_t)L.koff[(size_t)s] * 64;
+           e < (size_t)(L.koff[(size_t)s] + L.kmax[(size_t)s]) * 64; e++) {
+        const int j = L.col[e];
+        // (a padding slot's entries name the slot itself and are not read)
+        (*ccol)[e] = L.slot2orig[(size_t)j] < 0
+                         ? 0 : (unsigned short)((*cbase)[(size_t)(j >> 6)] + (j & 63));
+      }
+  }
+}
 
 template <typename T>
 static int balloc(T** p, size_t n) {
@@ -278,6 +509,8 @@ static BatchArgs batch_args(fc3d_hip_batch* b) {
   A.out_iter = b->out_iter;
   A.out_fp32_iter = b->out_fp32;
   A.out_residual = b->out_res;
+  A.cbase = b->d_cbase;
+  A.ccol = b->d_ccol;
   return A;
 }
 
@@ -303,6 +536,52 @@ static int ensure_fp32_batch(fc3d_hip_batch* b) {
   return 0;
 }
 
+// Reactions in LDS, 32 bytes a contact: two workgroups' a CU (what the waves'
+// registers allow) within its 160 KB.
+constexpr int BATCH_LDS_CONTACTS = 2048;
+constexpr int BATCH_QUAD_PROBLEMS = 2048;
+
+// lds_contacts: the largest problem's contacts if the quads may keep the
+// reactions in LDS (four waves a problem), else 0.
+static void launch_k_batch(const BatchArgs& A, const DevParams* prm, int wpp, int grid, int mixed,
+                           int lds_contacts, hipStream_t s) {
+  const dim3 g((unsigned)grid), t((unsigned)(64 * wpp));
+  const bool lds = wpp == 4 && lds_contacts > 0;
+  const size_t bytes = lds ? sizeof(double4) * (size_t)lds_contacts : 0;
+  void (*k)(BatchArgs, const DevParams*);
+  if (lds)
+    k = mixed ? k_batch<4, true, true> : k_batch<4, true, false>;
+  else if (wpp == 4)
+    k = mixed ? k_batch<4, false, true> : k_batch<4, false, false>;
+  else
+    k = mixed ? k_batch<1, false, true> : k_batch<1, false, false>;
+  hipLaunchKernelGGL(k, g, t, bytes, s, A, prm);
+}
+
+int launch_small_solve(const SweepPtrs<double>& P, const int* cptr, const int* cbase,
+                       const unsigned short* ccol, int nc, const DevParams* prm, SmallSolve* d,
+                       hipStream_t s) {
+  BatchArgs A;
+  std::memset(&A, 0, sizeof A);
+  A.P64 = P;
+  A.cptr = cptr;
+  A.problems = &d->problem;
+  A.order = &d->order;
+  A.nprob = 1;
+  A.counter = &d->counter;
+  A.out_info = &d->info;
+  A.out_iter = &d->iterations;
+  A.out_fp32_iter = &d->fp32_iterations;
+  A.out_residual = &d->residual;
+  A.out_incr = &d->incr;
+  A.cbase = cbase;
+  A.ccol = ccol;
+  hipLaunchKernelGGL((k_batch<8, true, false>), dim3(1), dim3(512), sizeof(double4) * (size_t)nc, s,
+                     A, prm);
+  FC3D_HIP_TRY(hipGetLastError());
+  return 0;
+}
+
 // Launches the persistent kernel with `wpp` waves per problem; grid = enough
 // workgroups to fill the device at the kernel's occupancy.
 static int launch_batch(fc3d_hip_batch* b, int wpp, int mixed) {
@@ -311,11 +590,8 @@ static int launch_batch(fc3d_hip_batch* b, int wpp, int mixed) {
   FC3D_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
   const int per_cu = wpp == 1 ? 8 : 2;  // 2 waves/SIMD at this kernel's register use
   const int grid = std::max(1, std::min(b->nprob, cus * per_cu));
-  const BatchArgs A = batch_args(b);
-  if (wpp == 4)
-    hipLaunchKernelGGL(k_batch<4>, dim3(grid), dim3(256), 0, b->stream, A, b->prm, mixed);
-  else
-    hipLaunchKernelGGL(k_batch<1>, dim3(grid), dim3(64), 0, b->stream, A, b->prm, mixed);
+  const int lds = b->max_nc <= BATCH_LDS_CONTACTS ? b->max_nc : 0;
+  launch_k_batch(batch_args(b), b->prm, wpp, grid, mixed, lds, b->stream);
   FC3D_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -416,10 +692,15 @@ int fc3d_hip_batch_create(int nprob, const int* nc, const int64_t* row_ptr,
   b->slot2orig = L.slot2orig;
   b->orig2slot = L.orig2slot;
   b->cptr = L.colour_slice_ptr;
+  std::vector<int> cbase;
+  std::vector<unsigned short> ccol;
+  b->max_nc = *std::max_element(b->nc.begin(), b->nc.end());
+  if (b->max_nc <= BATCH_LDS_CONTACTS) number_contacts(L, b->problems, &cbase, &ccol);
   std::vector<int> order((size_t)nprob);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return nc[x] > nc[y]; });
-  if ((rc = bupload(&b->len, L.len)) || (rc = bupload(&b->dpos, L.dpos)) ||
+  if ((rc = bupload(&b->d_cbase, cbase)) || (rc = bupload(&b->d_ccol, ccol)) ||
+      (rc = bupload(&b->len, L.len)) || (rc = bupload(&b->dpos, L.dpos)) ||
       (rc = bupload(&b->koff, L.koff)) || (rc = bupload(&b->kmax, L.kmax)) ||
       (rc = bupload(&b->col, L.col)) || (rc = bupload(&b->vals, L.vals)) ||
       (rc = bupload(&b->diag, L.diag)) || (rc = bupload(&b->q, L.q)) ||
@@ -451,6 +732,8 @@ void fc3d_hip_batch_destroy(fc3d_hip_batch* b) {
   for (void* p : ptrs)
     if (p) hipFree(p);
   b->transfer.release();
+  if (b->d_cbase) hipFree(b->d_cbase);
+  if (b->d_ccol) hipFree(b->d_ccol);
   if (b->stream) hipStreamDestroy(b->stream);
   delete b;
 }
@@ -549,6 +832,12 @@ int fc3d_hip_batch_solve(fc3d_hip_batch* b, const fc3d_hip_params* p, fc3d_hip_b
     set_error("fc3d_hip_batch_solve: schedule %d out of range [0, 2]", p->schedule);
     return NUMERICS_ERR_INVALID_ARGUMENT;
   }
+  // Few problems: quads, without the trial, whose 8 sweeps see the throughput
+  // of the start and not the slow problems that the launch ends with (it took
+  // one wave a problem where quads win).  ms one wave / quads, FP64: 1024
+  // problems 126 / 100, 2048 170 / 125, 4096 180 / 195; mixed: 68 / 51,
+  // 78 / 67, 97 / 99.
+  if (wpp == 0 && b->max_nc <= BATCH_LDS_CONTACTS && b->nprob <= BATCH_QUAD_PROBLEMS) wpp = 4;
   if (wpp == 0) {
     if (!b->tuned_wpp[mixed]) {
       double4* saved = nullptr;

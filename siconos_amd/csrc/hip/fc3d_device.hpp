@@ -829,14 +829,6 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
     if (!damped && P.formulation != 1)
       return nsn_newton_std_fp32<T>(lp, r, P, tol, rho, residual);
   }
-  if constexpr (sizeof(T) == 8) {
-    if (P.formulation != 1) {
-      double F2, nrel;
-      const int info = nsn_newton_std_fp64(lp, r, P, tol, rho, damped, &F2, &nrel);
-      *residual = sqrt(F2) * nrel;
-      return info;
-    }
-  }
   const T nq = qsqrt<T>(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
   T nrel = T(1);
   if (nq > num<T>::eps) nrel = qdiv<T>(nrel, nq);
@@ -987,68 +979,15 @@ __device__ __forceinline__ void keep_or_discard(const LocalProblem<T>& lp, T* r,
   }
 }
 
-// The damped Newton of the hybrid solver, of whose residual it reads only
-// whether it is a number: with the STD formulation in FP64 that is whether
-// |F|^2 is one (1 / |q| is at most 1 / DBL_EPSILON), and no root is taken.
-template <typename T>
-__device__ __forceinline__ int hybrid_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
-                                             T tol, const T* rho, T* res) {
-  if constexpr (sizeof(T) == 8) {
-    if (P.formulation != 1) {
-      double nrel;
-      return nsn_newton_std_fp64(lp, r, P, tol, rho, true, res, &nrel);
-    }
-  }
-  return nsn_newton<T>(lp, r, P, tol, rho, true, res);
-}
-
-// onecontact...c:920-1015
+// onecontact...c:920-1015 (the FP32 sweeps' form)
 template <typename T>
 __device__ int hybrid_solve(const LocalProblem<T>& lp, T* r, const LocalParams& P, T tol,
                             T* rho_pli, const T* rho, T* residual) {
   int info = -1;
   T bak[3] = {r[0], r[1], r[2]};
-  T res = T(0), cur;
-  if constexpr (sizeof(T) == 8) {
-    // the starting error matters only where the Newton solution is not
-    // accepted by its own error, so it is evaluated only there; the caller
-    // reads an accepted error only as a number not above 1 (the filter), which
-    // tol <= 1 bounds, so its root is taken only for a larger tol
-    if (P.hybrid_strategy == 2) {
-      info = hybrid_newton<T>(lp, r, P, tol, rho, &res);
-      const T nq = sqrt(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
-      T v[3];
-      local_velocity<T>(lp, r, v);
-      const T ue = unitary_error<T>(r, v, lp.mu);
-      auto error = [&]() {
-        const T x = sqrt(ue);
-        return nq > num<T>::eps ? x / nq : x;
-      };
-      const bool number = !(isnan(res) || isinf(res));
-      if (number && root_test(ue, nq > num<T>::eps ? tol * nq : tol,
-                              [&]() { return error() <= tol; })) {
-        *residual = tol <= T(1) ? tol : error();
-        return info;
-      }
-      const T e = error();
-      cur = compute_local_error<T>(lp, bak);
-      if (number && e <= cur) {
-        cur = e;
-        bak[0] = r[0]; bak[1] = r[1]; bak[2] = r[2];
-      } else {
-        r[0] = bak[0]; r[1] = bak[1]; r[2] = bak[2];
-      }
-      if (cur <= tol) {
-        *residual = cur;
-        return info;
-      }
-    } else {
-      cur = compute_local_error<T>(lp, r);
-    }
-  } else {
-    cur = compute_local_error<T>(lp, r);
-  }
-  if (sizeof(T) == 4 && P.hybrid_strategy == 2) {
+  T cur = compute_local_error<T>(lp, r);
+  T res = T(0);
+  if (P.hybrid_strategy == 2) {
     info = nsn_newton<T>(lp, r, P, tol, rho, true, &res);
     keep_or_discard<T>(lp, r, bak, tol, res, &cur);
     if (cur <= tol) {
@@ -1062,8 +1001,72 @@ __device__ int hybrid_solve(const LocalProblem<T>& lp, T* r, const LocalParams& 
     info = pli_solve<T>(lp, r, P.hybrid_max_iter, tol, rho_pli, &res);
     keep_or_discard<T>(lp, r, bak, tol, res, &cur);
     if (cur < tol) break;
-    info = hybrid_newton<T>(lp, r, P, tol, rho, &res);
+    info = nsn_newton<T>(lp, r, P, tol, rho, true, &res);
     keep_or_discard<T>(lp, r, bak, tol, res, &cur);
+  }
+  *residual = cur;
+  return info;
+}
+
+// The Newton solvers in FP64: 550 (onecontact...c:429-559), 551 (:710-854) and
+// the hybrid 565 (:920-1015), whose first and later Newton solves are one call
+// site: four inlined copies of the Newton loop did not fit the instruction
+// cache of a kernel that runs many sweeps (64 KB for two CUs).  The hybrid's
+// starting error is evaluated only where the first Newton solution is not
+// accepted by its own.  Of the Newton residual it reads only whether it is a
+// number, which with the STD formulation is whether |F|^2 is one (1 / |q| is
+// at most 1 / DBL_EPSILON).  An accepted error is returned as tol when tol <=
+// 1: the caller reads it as a number not above 1 (the filter).
+__device__ inline int newton_solvers_fp64(const LocalProblem<double>& lp, double* r,
+                                          const LocalParams& P, double tol, double* rho_pli,
+                                          const double* rho, double* residual) {
+  const bool hybrid = P.solver != 550 && P.solver != 551;
+  bool first = !hybrid || P.hybrid_strategy == 2;
+  int info = -1, loop = 0;
+  double bak[3] = {r[0], r[1], r[2]}, res = 0.0, cur = 0.0;
+  const double nq = sqrt(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
+  if (!first) cur = compute_local_error<double>(lp, r);
+  for (;;) {
+    if (!first) {
+      if (!(loop < P.hybrid_max_loop && cur >= tol)) break;
+      loop++;
+      info = pli_solve<double>(lp, r, P.hybrid_max_iter, tol, rho_pli, &res);
+      keep_or_discard<double>(lp, r, bak, tol, res, &cur);
+      if (cur < tol) break;
+    }
+    double nrel = 1.0;
+    const bool std_form = P.formulation != 1;
+    if (std_form)
+      info = nsn_newton_std_fp64(lp, r, P, tol, rho, P.solver != 550, &res, &nrel);
+    else
+      info = nsn_newton<double>(lp, r, P, tol, rho, P.solver != 550, &res);
+    if (!hybrid) {
+      *residual = std_form ? sqrt(res) * nrel : res;
+      return info;
+    }
+    double v[3];
+    local_velocity<double>(lp, r, v);
+    const double ue = unitary_error<double>(r, v, lp.mu);
+    auto error = [&]() {
+      const double x = sqrt(ue);
+      return nq > DBL_EPSILON ? x / nq : x;
+    };
+    const bool number = !(isnan(res) || isinf(res));
+    if (first && number && root_test(ue, nq > DBL_EPSILON ? tol * nq : tol,
+                                     [&]() { return error() <= tol; })) {
+      *residual = tol <= 1.0 ? tol : error();
+      return info;
+    }
+    const double e = error();
+    if (first) cur = compute_local_error<double>(lp, bak);
+    if (number && (e <= tol || e <= cur)) {
+      cur = e;
+      bak[0] = r[0]; bak[1] = r[1]; bak[2] = r[2];
+    } else {
+      r[0] = bak[0]; r[1] = bak[1]; r[2] = bak[2];
+    }
+    if (first && cur <= tol) break;
+    first = false;
   }
   *residual = cur;
   return info;
@@ -1086,6 +1089,8 @@ __device__ int local_solve(const LocalProblem<T>& lp, T* r, const LocalParams& P
     *residual = T(0);
     return 0;
   }
+  if constexpr (sizeof(T) == 8)
+    return newton_solvers_fp64(lp, r, P, tol, state_pli, rho, residual);
   if (P.solver == 550) return nsn_newton<T>(lp, r, P, tol, rho, false, residual);
   if (P.solver == 551) return nsn_newton<T>(lp, r, P, tol, rho, true, residual);
   return hybrid_solve<T>(lp, r, P, tol, state_pli, rho, residual);

@@ -25,6 +25,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "fc3d_batch.hpp"
 #include "fc3d_internal.hpp"
 #include "fc3d_accel.hpp"
 #include "fc3d_velocity.hpp"
@@ -645,6 +646,10 @@ struct fc3d_hip_problem {
   std::vector<int> orig2slot;
   std::vector<double> colour_bytes64, colour_bytes32;  // algorithmic bytes per colour pass
   std::vector<double> colour_nc;                       // contacts per colour
+  // small problems (SMALL_*): the one-workgroup solve
+  int* d_cbase = nullptr;
+  unsigned short* d_ccol = nullptr;
+  SmallSolve* d_small = nullptr;
   // device
   int *len = nullptr, *dpos = nullptr, *koff = nullptr, *kmax = nullptr, *col = nullptr;
   double *vals = nullptr, *diag = nullptr, *q = nullptr, *mu = nullptr, *pli = nullptr;
@@ -1619,6 +1624,50 @@ static int tune_schedule(fc3d_hip_problem* h, int phase, double norm_q, double l
   return 0;
 }
 
+// A small problem's plain FP64 solve runs whole in one workgroup (k_batch's
+// quads, reactions in LDS; the same sweeps and bits): no launch, no memory
+// round trip for a colour's reactions.  The two quads take a colour's slices
+// side by side, so it pays to three slices a colour.  us a sweep, this /
+// launches per colour: 40 contacts 47 / 75, 200 90 / 115, 500 (two slices)
+// 84 / 113, 1000 (three) 133 / 145 and 117 / 115, 1500 (four, five) 180 / 161
+// and 143 / 117.
+constexpr int SMALL_CONTACTS = 2000;  // 32 bytes of LDS each
+constexpr int SMALL_COLOUR_SLICES = 3;
+static bool small_solve(const fc3d_hip_problem* h, const fc3d_hip_params* p, bool observed) {
+  return h->d_small && p->schedule == 0 && p->precision == 0 && !p->velocity_form &&
+         p->accel_depth == 0 && p->freeze_contacts == 0 && p->warm_start <= 1 &&
+         !p->instrument && !observed && p->max_iter > 0;
+}
+
+static int solve_small(fc3d_hip_problem* h, const fc3d_hip_params* p, fc3d_hip_stats* s) {
+  int rc;
+  hipEvent_t t0, t1;
+  SmallSolve x;
+  std::memset(&x, 0, sizeof x);
+  x.problem = {0, h->ncolours, 0, h->nslices, h->norm_q};
+  FC3D_HIP_TRY(hipMemcpyAsync(h->d_small, &x, sizeof x, hipMemcpyHostToDevice, h->stream));
+  FC3D_HIP_TRY(hipEventCreate(&t0));
+  FC3D_HIP_TRY(hipEventCreate(&t1));
+  FC3D_HIP_TRY(hipEventRecord(t0, h->stream));
+  if ((rc = launch_small_solve(ptrs64(h, h->part), h->d_cps, h->d_cbase, h->d_ccol, h->nc, h->prm,
+                               h->d_small, h->stream)))
+    return rc;
+  FC3D_HIP_TRY(hipEventRecord(t1, h->stream));
+  FC3D_HIP_TRY(hipMemcpyAsync(&x, h->d_small, sizeof x, hipMemcpyDeviceToHost, h->stream));
+  FC3D_HIP_TRY(hipStreamSynchronize(h->stream));
+  float ms = 0.f;
+  hipEventElapsedTime(&ms, t0, t1);
+  hipEventDestroy(t0);
+  hipEventDestroy(t1);
+  s->solve_ms = ms;
+  s->iterations = x.iterations;
+  s->incr_error = x.incr;
+  s->residual = x.residual;
+  s->info = x.info;
+  s->schedule = FC3D_SCHEDULE_W4;
+  return 0;
+}
+
 // Frames layout detection: every contact's blocks must be H_a = [T | T S(l_a)]
 // and H_b = -[T | T S(l_b)] for one 3x3 T and lever arms l_a, l_b (a side
 // without a body is free).  l is read off the skew matrix sg T^-1 Rot, and the
@@ -1809,6 +1858,19 @@ int fc3d_hip_problem_create(int nc, const int64_t* row_ptr, const int64_t* col_i
   h->colour_nc.assign(h->colour_slice_ptr.size() - 1, 0.0);
   for (int c : h->colour) h->colour_nc[(size_t)c] += 1.0;
   build_dataflow(L, h->colour.data(), &h->dfh);
+  {
+    int widest = 0;
+    for (int c = 0; c < h->ncolours; c++)
+      widest = std::max(widest, h->colour_slice_ptr[(size_t)c + 1] - h->colour_slice_ptr[(size_t)c]);
+    if (nc <= SMALL_CONTACTS && widest <= SMALL_COLOUR_SLICES) {
+      std::vector<int> cbase;
+      std::vector<unsigned short> ccol;
+      number_contacts(L, {{0, h->ncolours, 0, h->nslices, 0.0}}, &cbase, &ccol);
+      if ((rc = dev_upload(&h->d_cbase, cbase)) || (rc = dev_upload(&h->d_ccol, ccol)) ||
+          (rc = dev_alloc(&h->d_small, 1)))
+        return fail(rc);
+    }
+  }
   std::vector<int2> planes((size_t)L.nslices);
   for (size_t k = 0; k < planes.size(); k++) planes[k] = make_int2(L.koff[k], L.kmax[k]);
   if ((rc = dev_upload(&h->d_planes, planes)) || (rc = dev_upload(&h->len, L.len)) || (rc = dev_upload(&h->dpos, L.dpos)) ||
@@ -1847,7 +1909,7 @@ void fc3d_hip_problem_destroy(fc3d_hip_problem* h) {
   free_stage_bufs(h);
   h->transfer.release();
   void* dfp[] = {h->dep_ptr, h->dep_idx, h->qlist, h->done,    h->df,    h->d_block_dst,
-                 h->d_o2s,    h->d_cps,    h->d_planes,   h->d_ba,   h->d_bb,   h->d_inc_ptr, h->d_inc, h->d_H,
+                 h->d_o2s,    h->d_cps,    h->d_planes, h->d_cbase, h->d_ccol, h->d_small,   h->d_ba,   h->d_bb,   h->d_inc_ptr, h->d_inc, h->d_H,
                  h->d_minv,   h->d_vfree,  h->d_V,    h->d_H32,     h->d_minv32, h->d_V32,
                  h->d_F,      h->d_F32,    h->d_frz,  h->d_le2,  h->d_fcnt,
                  h->d_fs,     h->d_bmark,  h->d_slice_colour, h->d_focus_cnt,
@@ -2331,6 +2393,10 @@ int fc3d_hip_solve_observed(fc3d_hip_problem* h, const fc3d_hip_params* p, fc3d_
   FC3D_HIP_TRY(hipMemcpyAsync(h->prm, &dp, sizeof dp, hipMemcpyHostToDevice, h->stream));
   if (p->warm_start == 1)
     FC3D_HIP_TRY(hipMemsetAsync(h->r, 0, sizeof(double4) * (size_t)h->nslots, h->stream));
+  if (small_solve(h, p, observer != nullptr)) {
+    h->accel_on = h->vel_on = h->focus_passes = 0;
+    return solve_small(h, p, s);
+  }
   const size_t ns = (size_t)h->nslots;
   hipLaunchKernelGGL(k_fill<double>, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, h->stream,
                      h->pli, 1.0, ns);

@@ -588,20 +588,36 @@ __device__ __forceinline__ void residual_slot(const SweepPtrs<double>& P, int s,
   double dg[9];
 #pragma unroll
   for (int e = 0; e < 9; e++) dg[e] = P.diag[(size_t)(s * 9 + e) * 64 + lane];
-  for (int k = 0; k < kmax; k++) {
-    if (k == dpos) mvp3x3<double>(dg, rv, u);
-    if (k < len) {
-      const size_t plane = (size_t)(koff + k);
-      const int j = P.col[plane * 64 + lane];
-      double w[9];
+  // four blocks and their reactions in flight: one by one, each block waits
+  // on two memory round trips
+  constexpr int U = 4;
+  const int* __restrict__ colp = P.col + (size_t)koff * 64 + lane;
+  const double* __restrict__ valp = P.vals + (size_t)koff * 9 * 64 + lane;
+  for (int k0 = 0; k0 < kmax; k0 += U) {
+    int j[U];
+    double w[U][9];
+    double4 rj[U];
 #pragma unroll
-      for (int e = 0; e < 9; e++) w[e] = P.vals[(plane * 9 + e) * 64 + lane];
-      const double4 rj = P.r[j];
-      const double v[3] = {rj.x, rj.y, rj.z};
-      mvp3x3<double>(w, v, u);
+    for (int t = 0; t < U; t++)
+      if (k0 + t < kmax) {
+        j[t] = colp[(size_t)(k0 + t) * 64];
+#pragma unroll
+        for (int e = 0; e < 9; e++) w[t][e] = valp[((size_t)(k0 + t) * 9 + e) * 64];
+      }
+#pragma unroll
+    for (int t = 0; t < U; t++)
+      if (k0 + t < kmax) rj[t] = P.r[j[t]];
+#pragma unroll
+    for (int t = 0; t < U; t++) {
+      if (k0 + t == dpos) mvp3x3<double>(dg, rv, u);
+      if (k0 + t < len) {
+        const double v[3] = {rj[t].x, rj[t].y, rj[t].z};
+        mvp3x3<double>(w[t], v, u);
+      }
     }
   }
-  if (dpos >= kmax) mvp3x3<double>(dg, rv, u);
+  // (the loop above ends at a multiple of U)
+  if (dpos >= (kmax + U - 1) / U * U) mvp3x3<double>(dg, rv, u);
   P.u[slot] = make_double4(u[0], u[1], u[2], 0.0);
   *e2 = unitary_error<double>(rv, u, P.mu[slot]);
   *r2 = rv[0] * rv[0] + rv[1] * rv[1] + rv[2] * rv[2];

@@ -109,3 +109,55 @@ def test_full_4096_problem_launch_converges_everywhere(oracle, batch4096, precis
         e, _ = oracle.compute_error(W, q, mu, r[3 * off[k]:3 * off[k + 1]])
         assert e <= 1e-6, (k, e)
         assert e == pytest.approx(res[k], rel=1e-9)
+
+
+@pytest.mark.parametrize("sizes", [(1, 2), (63, 64, 65), (513, 40), (2048, 8), (2049, 8)])
+@pytest.mark.parametrize("mode", [1, 2])
+def test_quads_at_their_edges(oracle, sizes, mode):
+    """Four waves a problem at the edges of a slice, of the reactions' place in
+    LDS (2048 contacts) and beyond it, with rows longer than the 16 planes a
+    lane holds, bit for bit per problem."""
+    probs = []
+    for k, n in enumerate(sizes):
+        nb = max(3, n // 6)  # ~24 blocks a row
+        while n > nb * (nb - 1) // 2:
+            nb += 1
+        g = N.generate_random_pairs(nb, n, 0.1, 0.9, 70 + k)
+        probs.append((g.W, g.q, g.mu))
+    B = N.Batch(probs)
+    s, info, it, res = B.solve(N.hip_params(tol=1e-4, max_iter=25, warm_start=1, schedule=2,
+                                            error_evaluation=mode))
+    order, r = B.order(), B.reaction()
+    for (W, q, mu), a, b, n in zip(probs, B.offsets[:-1], B.offsets[1:], it):
+        _, ro, _, _, _ = oracle.nsgs(W, q, mu, tol=1e-30, max_iter=int(n), order=order[a:b] - a)
+        np.testing.assert_array_equal(r[3 * a:3 * b], ro)
+
+
+@pytest.mark.parametrize("nc", [1, 64, 150, 400])
+def test_small_problem_in_one_workgroup(oracle, nc):
+    """A small problem's plain solve (one workgroup) against the oracle in the
+    same order and against one launch per colour: the same bits and sweeps in
+    every evaluation mode, from the resident reaction too."""
+    nb = max(3, int(nc * 0.45))
+    while nc > nb * (nb - 1) // 2:
+        nb += 1
+    g = N.generate_random_pairs(nb, nc, 0.2, 0.5, 5)
+    P = N.HipProblem(g.W, g.q, g.mu)
+    start = np.abs(np.random.default_rng(1).normal(size=3 * nc))
+    for mode in (0, 1, 2, 3):
+        out = []
+        for schedule in (0, 1):
+            P.set_reaction(start)
+            s = P.solve(N.hip_params(tol=1e-5, max_iter=40, schedule=schedule,
+                                     error_evaluation=mode, error_frequency=3))
+            out.append((P.reaction(), s.iterations, s.info, s.residual, s.incr_error))
+        np.testing.assert_array_equal(out[0][0], out[1][0])
+        assert out[0][1:3] == out[1][1:3]
+        for a, b in zip(out[0][3:], out[1][3:]):
+            assert a == b or a == pytest.approx(b, rel=1e-12)
+    _, ro, _, it, _ = oracle.nsgs(g.W, g.q, g.mu, tol=1e-5, max_iter=40, order=P.order(),
+                                  reaction=start)
+    P.set_reaction(start)
+    s = P.solve(N.hip_params(tol=1e-5, max_iter=40))
+    assert s.iterations == it
+    np.testing.assert_array_equal(P.reaction(), ro)
