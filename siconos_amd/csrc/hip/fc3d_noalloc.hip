@@ -44,9 +44,27 @@ static int scratch_on(int device, double** out) {
   return 0;
 }
 
-// Row ranges and column indices are checked against nnzb and nc: a row with
-// an entry outside them gets a NaN velocity (and so a NaN error) instead of
+// The row sum of contact i, block by block in the stored order.  Row ranges
+// and column indices are checked against nnzb and nc: a row with an entry
+// outside them is bad, and gets a NaN velocity (and so a NaN error) instead of
 // reading out of bounds.
+__device__ __forceinline__ void add_block(const double* w, const double* __restrict__ r, int64_t j,
+                                          double* u) {
+  const double v[3] = {r[3 * j], r[3 * j + 1], r[3 * j + 2]};
+  mvp3x3<double>(w, v, u);
+}
+
+// One wave per 64 contacts.  Their rows are one range of the CSR, which the
+// wave walks CSR_CHUNK blocks at a time: coalesced 512-byte loads of the
+// blocks into LDS, a lane per block for its products with the neighbour's
+// reaction (every gather of a chunk in flight), then a lane per row adds its
+// row's products in their order.  HBM bounds it (0.85 GB for 1M contacts with
+// 10.5M blocks): 1.8 TB/s when a lane walked its own row, 72 bytes in another
+// 128-byte line than its neighbours at every step (483 us a call, both
+// kernels), 4.1 TB/s so (208 us; a copy reaches 5.1).  A wave with a bad row
+// walks its rows from memory: every form of row pointers that was accepted
+// still is.
+constexpr int CSR_CHUNK = 128;
 __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
                                                       const int64_t* __restrict__ rp,
                                                       const int64_t* __restrict__ ci,
@@ -56,12 +74,70 @@ __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
                                                       const double* __restrict__ r,
                                                       double* __restrict__ u_out,
                                                       double* __restrict__ part) {
+  __shared__ double sblk[4][CSR_CHUNK * 9];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double e2 = 0.0, r2 = 0.0, u2 = 0.0;
+  double u[3] = {0.0, 0.0, 0.0};
+  int64_t k0 = 0, k1 = 0;
+  bool bad = false;
   if (i < nc) {
-    double u[3] = {q[3 * (size_t)i], q[3 * (size_t)i + 1], q[3 * (size_t)i + 2]};
-    const int64_t k0 = rp[i], k1 = rp[i + 1];
-    bool bad = k0 < 0 || k1 > nnzb || k1 < k0;
+#pragma unroll
+    for (int e = 0; e < 3; e++) u[e] = q[3 * (size_t)i + e];
+    k0 = rp[i];
+    k1 = rp[i + 1];
+    bad = k0 < 0 || k1 > nnzb || k1 < k0;
+  }
+  // the wave's range, when its rows follow each other inside [0, nnzb]
+  const int last = min(63, nc - 1 - (i - lane));  // last lane with a row (< 0: none)
+  const bool plain = __builtin_amdgcn_ballot_w64(bad) == 0;
+  const int64_t kb = __shfl(k0, 0, 64), ke = last >= 0 ? __shfl(k1, last, 64) : 0;
+  if (plain && last >= 0) {
+    int64_t k = k0;
+    for (int64_t c0 = kb; c0 < ke; c0 += CSR_CHUNK) {
+      const int n = (int)min((int64_t)CSR_CHUNK, ke - c0);
+      const double* __restrict__ src = blocks + 9 * c0;
+      double t[CSR_CHUNK * 9 / 64], v[CSR_CHUNK / 64][3];
+      int64_t jc[CSR_CHUNK / 64];
+#pragma unroll
+      for (int x = 0; x < CSR_CHUNK / 64; x++)
+        jc[x] = x * 64 + lane < n ? ci[c0 + x * 64 + lane] : 0;
+#pragma unroll
+      for (int x = 0; x < CSR_CHUNK * 9 / 64; x++)
+        if (x * 64 + lane < 9 * n) t[x] = src[x * 64 + lane];
+#pragma unroll
+      for (int x = 0; x < CSR_CHUNK / 64; x++) {
+        const bool ok = jc[x] >= 0 && jc[x] < nc;
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+          const double y = r[3 * (size_t)(ok ? jc[x] : 0) + e];
+          v[x][e] = ok ? y : NAN;  // a column out of range: the row is NaN
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < CSR_CHUNK * 9 / 64; x++)
+        if (x * 64 + lane < 9 * n) sblk[wave][x * 64 + lane] = t[x];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int x = 0; x < CSR_CHUNK / 64; x++)
+        if (x * 64 + lane < n) {
+          double* b = &sblk[wave][9 * (x * 64 + lane)];
+#pragma unroll
+          for (int e = 0; e < 9; e++) b[e] = b[e] * v[x][e / 3];
+        }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      // u += W r_j as mvp3x3 adds it: column after column
+      for (const int64_t stop = min(k1, c0 + n); k < stop; k++) {
+        const double* b = &sblk[wave][9 * (int)(k - c0)];
+#pragma unroll
+        for (int e = 0; e < 9; e++) u[e % 3] += b[e];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();  // the chunk is read before the next one lands
+    }
+  } else if (i < nc) {
     for (int64_t k = bad ? k1 : k0; k < k1; k++) {
       const int64_t j = ci[k];
       if (j < 0 || j >= nc) {
@@ -71,9 +147,10 @@ __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
       double w[9];
 #pragma unroll
       for (int e = 0; e < 9; e++) w[e] = blocks[9 * k + e];
-      const double v[3] = {r[3 * j], r[3 * j + 1], r[3 * j + 2]};
-      mvp3x3<double>(w, v, u);
+      add_block(w, r, j, u);
     }
+  }
+  if (i < nc) {
     if (bad) u[0] = u[1] = u[2] = NAN;
 #pragma unroll
     for (int e = 0; e < 3; e++) u_out[3 * (size_t)i + e] = u[e];

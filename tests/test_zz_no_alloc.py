@@ -93,3 +93,44 @@ def test_no_alloc_residual_refuses_sizes_beyond_its_scratch():
     rc = lib.fc3d_hip_compute_error_device(g.nc, 0, p, p, p, p, p, p, -1.0, p, p, 0, None)
     assert rc == -2
     d.free()
+
+
+@pytest.mark.parametrize("nc", [1, 63, 64, 65, 130, 300])
+def test_no_alloc_residual_rows_of_every_length(nc):
+    """Rows of 0 to 300 blocks (several of the kernel's chunks, a wave's rows
+    ending inside one), then one row with a column out of range and one with a
+    range past the end: those rows are NaN and the others keep their bits."""
+    rng = np.random.default_rng(nc)
+    per = rng.integers(0, 8, nc)
+    per[rng.integers(nc)] = 300
+    rp = np.concatenate([[0], np.cumsum(per)])
+    ci = rng.integers(0, nc, rp[-1])
+    blocks = rng.normal(size=(rp[-1], 9))
+    q, r = rng.normal(size=3 * nc), rng.normal(size=3 * nc)
+    W = N.SparseBlock3(rp, ci, blocks.reshape(-1))
+    rc, u, err = _device_call(W, q, np.full(nc, 0.4), r, 1.0)
+    want = q.copy().reshape(-1, 3)
+    for i in range(nc):
+        for k in range(rp[i], rp[i + 1]):
+            for j in range(3):  # column after column, as mvp3x3
+                want[i] += blocks[k, 3 * j:3 * j + 3] * r[3 * ci[k] + j]
+    assert rc == 0 and np.isfinite(err)
+    np.testing.assert_array_equal(u, want.reshape(-1))
+    row = int(np.argmax(per))
+    bad = ci.copy()
+    bad[rp[row] + 5] = nc
+    rc, u, err = _device_call(N.SparseBlock3(rp, bad, blocks.reshape(-1)), q, np.full(nc, 0.4), r,
+                              1.0)
+    keep = np.repeat(np.arange(nc) != row, 3)
+    assert rc == 0 and np.isnan(err) and np.isnan(u[~keep]).all()
+    np.testing.assert_array_equal(u[keep], want.reshape(-1)[keep])
+    past = W.row_ptr.copy()
+    past[nc] += 1
+    short = N.SparseBlock3(past, ci, blocks.reshape(-1))
+    type(short).nnzb = property(lambda s: int(rp[-1]))
+    try:
+        rc, u, err = _device_call(short, q, np.full(nc, 0.4), r, 1.0)
+    finally:
+        type(short).nnzb = property(lambda s: int(s.row_ptr[-1]))
+    assert rc == 0 and np.isnan(err) and np.isnan(u[-3:]).all()
+    np.testing.assert_array_equal(u[:-3], want.reshape(-1)[:-3])
