@@ -67,8 +67,9 @@ FC3D_API int fc2d_hip_get_velocity(fc2d_hip_problem* h, double* velocity);
  *     runs the whole solve, colours separated by workgroup barriers;
  *   FC2D_SCHEDULE_PER_COLOUR: one thread per contact across the GPU, one
  *     launch per colour, sweeps replayed from a captured graph;
- *   FC2D_SCHEDULE_AUTO: per colour when some colour holds more than 2048
- *     contacts, one workgroup otherwise. */
+ *   FC2D_SCHEDULE_AUTO: one workgroup up to 9200 contacts (its LDS then holds
+ *     the reactions); beyond, per colour when some colour holds more than
+ *     2048 contacts, else one workgroup. */
 enum { FC2D_SCHEDULE_AUTO = 0, FC2D_SCHEDULE_ONE_WORKGROUP = 1, FC2D_SCHEDULE_PER_COLOUR = 2 };
 
 typedef struct fc2d_hip_params {

@@ -4,7 +4,8 @@
 // contact graph one after the other, in one of two schedules:
 //   one workgroup: one launch of 1024 threads runs the whole solve, colours
 //     separated by workgroup barriers, each thread taking the colour's
-//     contacts in strides; the light error, the LIGHT_WITH_FULL_FINAL
+//     contacts in strides (the reactions in LDS while they fit:
+//     k_fc2d_nsgs_lds); the light error, the LIGHT_WITH_FULL_FINAL
 //     tolerance logic and fc2d_compute_error (fc2d_compute_error.c:104-148)
 //     run in the same kernel, so a solve has no host round trip;
 //   per colour: one thread per contact over the whole GPU, one launch per
@@ -222,12 +223,16 @@ __global__ __launch_bounds__(FC2D_THREADS) void k_fc2d_error(Fc2dArgs A, double*
 // The light error and the tolerance logic after a sweep (fc2d_nsgs.c:136-142,
 // 191-228), for the light modes.  All threads of the workgroup call it and
 // get the same results.
-__device__ void end_of_sweep(const Fc2dArgs& A, double* sh, int mode, double tol,
-                             double* tolerance, double* error, int* notconv, int* vel) {
+// r: the current reactions (A.r, or a copy of them in LDS, which `flush`
+// writes to A.r before the full error reads them there).
+template <typename Flush>
+__device__ void end_of_sweep(const Fc2dArgs& A, const double* r, Flush flush, double* sh, int mode,
+                             double tol, double* tolerance, double* error, int* notconv,
+                             int* vel) {
   double l = 0.0, r2 = 0.0;
   for (int s = threadIdx.x; s < A.nc; s += FC2D_THREADS) {
     l += A.light[s];
-    r2 += A.r[2 * s] * A.r[2 * s] + A.r[2 * s + 1] * A.r[2 * s + 1];
+    r2 += r[2 * s] * r[2 * s] + r[2 * s + 1] * r[2 * s + 1];
   }
   l = block_sum(l, sh);
   r2 = block_sum(r2, sh);
@@ -241,6 +246,7 @@ __device__ void end_of_sweep(const Fc2dArgs& A, double* sh, int mode, double tol
     *notconv = 1;
     if (err < *tolerance) {
       *notconv = 0;
+      flush();
       const double abs_err = full_error(A, sh);
       *vel = 1;
       if (abs_err > tol) {
@@ -272,9 +278,115 @@ __global__ __launch_bounds__(FC2D_THREADS) void k_fc2d_nsgs(Fc2dArgs A, int iter
       }
       __syncthreads();  // the next colour reads this colour's reactions
     }
-    if (light_mode) end_of_sweep(A, sh, mode, tol, &tolerance, &error, &notconv, &vel);
+    if (light_mode)
+      end_of_sweep(A, A.r, [] {}, sh, mode, tol, &tolerance, &error, &notconv, &vel);
     __syncthreads();
   }
+  if (mode == SICONOS_NSGS_ERROR_EVALUATION_LIGHT_WITH_FULL_FINAL) {
+    error = full_error(A, sh);
+    vel = 1;
+    notconv = error < tol ? 0 : 1;
+  }
+  if (threadIdx.x == 0) {
+    out->iterations = iter;
+    out->notconv = notconv;
+    out->velocity_set = vel;
+    out->error = error;
+  }
+}
+
+// The one-workgroup solve with the reactions in LDS (problems of up to
+// FC2D_LDS_CONTACTS contacts), over a layout of its own: a colour's contacts,
+// longest rows first, in groups of 64, one group a wave's step and one contact
+// a lane; both rows' entries in planes [k][row][64] (values, and the entry's
+// place in LDS as 16 bits), so that every load is one coalesced line run and
+// none depends on another; per-contact data in the same lane order.  Padded
+// entries are zeros that read a zero cell, and so are the own-contact entries
+// that only add w * 0.  A sweep's 2 MB come from one XCD's L2 over the CU's 64
+// bytes a cycle (~14 us of the 40 us a sweep of a 7056-contact layer); with
+// the reactions and rows in HBM and a launch per colour it took 71 us: every
+// colour waited on a launch and three dependent round trips.
+constexpr int FC2D_LDS_CONTACTS = 9200;  // 144 KB of the CU's 160
+
+struct Fc2dGroups {
+  const int* gptr;             // colour -> group range
+  const int2* planes;          // per group: first plane, number of planes
+  const int* slot;             // [group][64], -1 for padding
+  const double* con;           // [group][8][64]: diag (4), det, q (2), mu
+  const unsigned short* place;  // [plane][2][64]
+  const double* val;           // [plane][2][64]
+};
+
+__global__ __launch_bounds__(FC2D_THREADS) void k_fc2d_nsgs_lds(Fc2dArgs A, Fc2dGroups G,
+                                                               int itermax, double tol, int mode,
+                                                               Fc2dOut* out) {
+  __shared__ double sh[FC2D_THREADS / 64];
+  __shared__ double r[2 * FC2D_LDS_CONTACTS + 1];
+  constexpr int C = 6;  // planes in flight: 24 loads a lane
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  for (int i = threadIdx.x; i < 2 * A.nc; i += FC2D_THREADS) r[i] = A.r[i];
+  if (threadIdx.x == 0) r[2 * A.nc] = 0.0;  // what padded entries read
+  __syncthreads();
+  auto flush = [&] {
+    for (int i = threadIdx.x; i < 2 * A.nc; i += FC2D_THREADS) A.r[i] = r[i];
+    __syncthreads();
+  };
+  int iter = 0, notconv = 1, vel = 0;
+  double error = INFINITY, tolerance = tol;
+  const bool light_mode = is_light(mode);
+  while (iter < itermax && notconv) {
+    ++iter;
+    for (int c = 0; c < A.ncolours; c++) {
+      for (int g = G.gptr[c] + wave; g < G.gptr[c + 1]; g += FC2D_THREADS / 64) {
+        const int2 pl = G.planes[g];
+        const int p0 = __builtin_amdgcn_readfirstlane(pl.x),
+                  np = __builtin_amdgcn_readfirstlane(pl.y);
+        const unsigned short* __restrict__ place = G.place + (size_t)p0 * 128;
+        const double* __restrict__ val = G.val + (size_t)p0 * 128;
+        const int slot = G.slot[g * 64 + lane];
+        const double* __restrict__ con = G.con + (size_t)g * 512 + lane;
+        double W[4], q[2];
+#pragma unroll
+        for (int e = 0; e < 4; e++) W[e] = con[e * 64];
+        const double det = con[256], mu = con[448];
+        q[0] = con[320];
+        q[1] = con[384];
+        const bool dot = A.row_mode == FC2D_ROWS_DOT;
+        double y[2] = {dot ? 0.0 : q[0], dot ? 0.0 : q[1]};
+        for (int k0 = 0; k0 < np; k0 += C) {
+          unsigned short j[C][2];
+          double w[C][2];
+#pragma unroll
+          for (int k = 0; k < C; k++)
+            if (k0 + k < np)
+#pragma unroll
+              for (int i = 0; i < 2; i++) {
+                j[k][i] = (place + (k0 + k) * 128 + i * 64)[lane];
+                w[k][i] = (val + (k0 + k) * 128 + i * 64)[lane];
+              }
+#pragma unroll
+          for (int k = 0; k < C; k++)
+            if (k0 + k < np)
+#pragma unroll
+              for (int i = 0; i < 2; i++) y[i] += w[k][i] * r[j[k][i]];
+        }
+        if (slot < 0) continue;
+        const double ql[2] = {dot ? q[0] + y[0] : y[0], dot ? q[1] + y[1] : y[1]};
+        const double o0 = r[2 * slot], o1 = r[2 * slot + 1];
+        double P[2] = {o0, o1};
+        local_solve(W, det, ql, mu, P);
+        const double x0 = o0 - P[0], x1 = o1 - P[1];
+        A.light[slot] = x0 * x0 + x1 * x1;
+        r[2 * slot] = P[0];
+        r[2 * slot + 1] = P[1];
+      }
+      __syncthreads();  // the next colour reads this colour's reactions
+    }
+    if (light_mode)
+      end_of_sweep(A, r, flush, sh, mode, tol, &tolerance, &error, &notconv, &vel);
+    __syncthreads();
+  }
+  flush();
   if (mode == SICONOS_NSGS_ERROR_EVALUATION_LIGHT_WITH_FULL_FINAL) {
     error = full_error(A, sh);
     vel = 1;
@@ -325,7 +437,8 @@ __global__ __launch_bounds__(FC2D_THREADS) void k_fc2d_end_sweep(Fc2dArgs A, Fc2
   const int iter = st->iter + 1, mode = st->mode;
   int notconv = 1, vel = st->vel;
   double error = st->error, tolerance = st->tolerance;
-  if (is_light(mode)) end_of_sweep(A, sh, mode, st->tol, &tolerance, &error, &notconv, &vel);
+  if (is_light(mode))
+    end_of_sweep(A, A.r, [] {}, sh, mode, st->tol, &tolerance, &error, &notconv, &vel);
   __syncthreads();  // every thread has read st
   if (threadIdx.x == 0) {
     st->iter = iter;
@@ -383,6 +496,11 @@ struct fc2d_hip_problem {
   hipGraphExec_t graph = nullptr;  // FC2D_GRAPH_SWEEPS sweeps of it
   std::vector<int> hcptr;          // colour -> slot range, on the host
   hipEvent_t ev[2] = {nullptr, nullptr};
+  // the one-workgroup solve's layout, when the reactions fit LDS
+  int *g_ptr = nullptr, *g_slot = nullptr;
+  int2* g_planes = nullptr;
+  double *g_con = nullptr, *g_val = nullptr;
+  unsigned short* g_place = nullptr;
 
   Fc2dArgs args() const {
     Fc2dArgs a;
@@ -410,14 +528,82 @@ struct fc2d_hip_problem {
 // flag after each replay; sweeps after the stop return at once.
 constexpr int FC2D_GRAPH_SWEEPS = 16;
 
-// The schedule a solve uses: the requested one, or automatically one launch
-// per colour when some colour holds more contacts than one workgroup sweeps
-// in two strides (below that, one workgroup's barriers cost less than the
-// launches).  -1 for an unknown request.
+// Builds Fc2dGroups for a problem in slot order (rows srp, places src, values
+// srv).  The order inside a colour is free: its contacts share no row entry.
+static int build_groups(fc2d_hip_problem* h, const std::vector<int>& cptr,
+                        const std::vector<int>& srp, const std::vector<int>& src,
+                        const std::vector<double>& srv, const std::vector<double>& sdiag,
+                        const std::vector<double>& sdet, const std::vector<double>& sq,
+                        const std::vector<double>& smu) {
+  const unsigned short zero = (unsigned short)(2 * h->nc);
+  std::vector<int> gptr(1, 0), slots;
+  std::vector<int2> planes;
+  std::vector<double> con, val;
+  std::vector<unsigned short> place;
+  // entries of a row that the sweep adds: own-contact ones only as w * 0
+  auto own = [&](int s, int e) { return src[(size_t)e] >> 1 == s; };
+  auto row_len = [&](int s, int i) {
+    int n = 0;
+    for (int e = srp[2 * (size_t)s + i]; e < srp[2 * (size_t)s + i + 1]; e++)
+      n += h->own_zero || !own(s, e);
+    return n;
+  };
+  int np = 0;
+  for (int c = 0; c < h->ncolours; c++) {
+    std::vector<std::pair<int, int>> m;  // (-longest row, slot)
+    for (int s = cptr[(size_t)c]; s < cptr[(size_t)c + 1]; s++)
+      m.push_back({-std::max(row_len(s, 0), row_len(s, 1)), s});
+    std::sort(m.begin(), m.end());
+    for (size_t b = 0; b < m.size(); b += 64) {
+      const int k = -m[b].first;
+      const size_t g = planes.size();
+      planes.push_back(make_int2(np, k));
+      slots.resize(64 * (g + 1), -1);
+      con.resize(512 * (g + 1), 0.0);
+      place.resize((size_t)(np + k) * 128, zero);
+      val.resize((size_t)(np + k) * 128, 0.0);
+      for (size_t l = 0; l < 64 && b + l < m.size(); l++) {
+        const int s = m[b + l].second;
+        slots[64 * g + l] = s;
+        double* cg = con.data() + 512 * g + l;
+        for (int e = 0; e < 4; e++) cg[64 * e] = sdiag[4 * (size_t)s + (size_t)e];
+        cg[256] = sdet[(size_t)s];
+        cg[320] = sq[2 * (size_t)s];
+        cg[384] = sq[2 * (size_t)s + 1];
+        cg[448] = smu[(size_t)s];
+        for (int i = 0; i < 2; i++) {
+          size_t t = (size_t)np * 128 + (size_t)i * 64 + l;
+          for (int e = srp[2 * (size_t)s + i]; e < srp[2 * (size_t)s + i + 1]; e++) {
+            if (own(s, e) && !h->own_zero) continue;
+            place[t] = own(s, e) ? zero : (unsigned short)src[(size_t)e];
+            val[t] = srv[(size_t)e];
+            t += 128;
+          }
+        }
+      }
+      np += k;
+    }
+    gptr.push_back((int)planes.size());
+  }
+  int rc;
+  if ((rc = dev_upload(&h->g_ptr, gptr)) || (rc = dev_upload(&h->g_slot, slots)) ||
+      (rc = dev_upload(&h->g_planes, planes)) || (rc = dev_upload(&h->g_con, con)) ||
+      (rc = dev_upload(&h->g_val, val)) || (rc = dev_upload(&h->g_place, place)))
+    return rc;
+  return 0;
+}
+
+// The schedule a solve uses: the requested one, or automatically one workgroup
+// when the reactions fit its LDS (us a sweep, one workgroup / per colour: 31
+// contacts 9.5 / 31, 431 15 / 47, 2070 19 / 62, 7056 40 / 71, 8985 49 / 73),
+// else one launch per colour when some colour holds more contacts than one
+// workgroup sweeps in two strides (below that, one workgroup's barriers cost
+// less than the launches).  -1 for an unknown request.
 static int fc2d_schedule(const fc2d_hip_problem* h, int requested) {
   if (requested == FC2D_SCHEDULE_ONE_WORKGROUP || requested == FC2D_SCHEDULE_PER_COLOUR)
     return requested;
   if (requested != FC2D_SCHEDULE_AUTO) return -1;
+  if (h->g_ptr) return FC2D_SCHEDULE_ONE_WORKGROUP;
   int widest = 0;
   for (size_t c = 0; c + 1 < h->hcptr.size(); c++)
     widest = std::max(widest, h->hcptr[c + 1] - h->hcptr[c]);
@@ -473,6 +659,9 @@ void fc2d_hip_problem_destroy(fc2d_hip_problem* h) {
     void* ptrs[] = {h->cptr, h->rp, h->rc,    h->rv,  h->diag, h->det, h->q,
                     h->mu,   h->r,  h->u,     h->light, h->err, h->out, h->st};
     for (void* p : ptrs)
+      if (p) hipFree(p);
+    void* groups[] = {h->g_ptr, h->g_slot, h->g_planes, h->g_con, h->g_val, h->g_place};
+    for (void* p : groups)
       if (p) hipFree(p);
     for (hipEvent_t e : h->ev)
       if (e) hipEventDestroy(e);
@@ -617,6 +806,11 @@ int fc2d_hip_problem_create(int nc, const int64_t* row_ptr, const int64_t* cols,
     return rc;
   }
   h->hcptr = cptr;
+  if (nc <= FC2D_LDS_CONTACTS &&
+      (rc = build_groups(h, cptr, srp, src, srv, sdiag, sdet, sq, smu))) {
+    fc2d_hip_problem_destroy(h);
+    return rc;
+  }
   if (hipMalloc(&h->err, sizeof(double)) != hipSuccess ||
       hipMalloc(&h->out, sizeof(Fc2dOut)) != hipSuccess ||
       hipMalloc(&h->st, sizeof(Fc2dState)) != hipSuccess) {
@@ -739,8 +933,14 @@ int fc2d_hip_solve(fc2d_hip_problem* h, const fc2d_hip_params* p, fc2d_hip_stats
                        h->out);
   } else {
     FC3D_HIP_TRY(hipEventRecord(h->ev[0], h->stream));
-    hipLaunchKernelGGL(k_fc2d_nsgs, dim3(1), dim3(FC2D_THREADS), 0, h->stream, h->args(),
-                       p->max_iter, p->tol, p->error_evaluation, h->out);
+    if (h->g_ptr) {
+      const Fc2dGroups g = {h->g_ptr, h->g_planes, h->g_slot, h->g_con, h->g_place, h->g_val};
+      hipLaunchKernelGGL(k_fc2d_nsgs_lds, dim3(1), dim3(FC2D_THREADS), 0, h->stream, h->args(), g,
+                         p->max_iter, p->tol, p->error_evaluation, h->out);
+    } else {
+      hipLaunchKernelGGL(k_fc2d_nsgs, dim3(1), dim3(FC2D_THREADS), 0, h->stream, h->args(),
+                         p->max_iter, p->tol, p->error_evaluation, h->out);
+    }
   }
   FC3D_HIP_TRY(hipGetLastError());
   FC3D_HIP_TRY(hipEventRecord(h->ev[1], h->stream));

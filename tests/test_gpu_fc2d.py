@@ -7,11 +7,14 @@ counterpart (test_fc2d_gpu.c) runs the same collection.  The GPU sweeps in
 colour order; the oracle run in that order gives the same reactions bit for
 bit and the same iteration count.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from conftest import FC2D_COLLECTION, fixture_file
 from oracle import pyoracle as O
+from siconos_amd import capi
 from siconos_amd import numerics as N
 
 pytestmark = pytest.mark.gpu
@@ -217,3 +220,47 @@ def test_edge_cases_through_the_driver(lib, tmp_path, case):
         s = H.solve(max_iter=10000, tol=1e-5, error_evaluation=2, schedule=sched)
         assert s.info == 0 and s.iterations == it
         np.testing.assert_array_equal(H.reaction(), r)
+
+
+@pytest.mark.parametrize("nc", [1, 64, 65, 700, 9200, 9201])
+@pytest.mark.parametrize("row_mode,own_zero", [(0, 0), (0, 1), (1, 0)])
+def test_one_workgroup_at_the_edges_of_its_lds(lib, nc, row_mode, own_zero):
+    """A chain of contacts (every third one also tied to the first, so that
+    rows differ in length) up to and beyond the size whose reactions fit LDS:
+    both schedules give the same bits, from a start that is not zero."""
+    rng = np.random.default_rng(nc)
+    rows = [[] for _ in range(nc)]
+    for c in range(nc):
+        for d in {c, c - 1, c + 1} | ({0} if c % 3 == 0 and c < 90 else set()):
+            if 0 <= d < nc:
+                rows[c].append(d)
+    for c in range(3, min(nc, 90), 3):
+        rows[0].append(c)
+    rp, cols, vals, diag = [0], [], [], []
+    for c in range(nc):
+        blk = {d: rng.normal(size=(2, 2)) * 0.1 + (3.0 * np.eye(2) if d == c else 0.0)
+               for d in sorted(set(rows[c]))}
+        for i in range(2):
+            for d, b in blk.items():
+                for k in range(2):
+                    cols.append(2 * d + k)
+                    vals.append(b[i, k])
+            rp.append(len(cols))
+        diag.append(blk[c].reshape(-1, order="F"))
+    rp, cols = np.array(rp, dtype=np.int64), np.array(cols, dtype=np.int64)
+    vals, diag = np.array(vals), np.ascontiguousarray(np.concatenate(diag))
+    q, mu = rng.normal(size=2 * nc), rng.uniform(0.1, 0.8, nc)
+    h = C.c_void_p()
+    assert lib.fc2d_hip_problem_create(nc, N.lptr(rp), N.lptr(cols), N.dptr(vals), row_mode,
+                                       own_zero, N.dptr(diag), N.dptr(q), N.dptr(mu), 0,
+                                       C.byref(h)) == 0, capi.last_error()
+    P = N.Fc2dHipProblem.__new__(N.Fc2dHipProblem)
+    P._lib, P.nc, P._h = lib, nc, h
+    start = np.abs(rng.normal(size=2 * nc))
+    out = []
+    for schedule in (1, 2):
+        P.set_reaction(start)
+        s = P.solve(max_iter=30, tol=1e-9, schedule=schedule)
+        out.append((P.reaction(), P.velocity(), s.iterations, s.residual, s.info))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
