@@ -3,13 +3,21 @@
 // MLP 22 -> 128 -> 128 -> 128 -> 3 with GELU.  Every product runs on the
 // matrix cores as v_mfma_f32_16x16x16bf16_1k (BF16 operands, FP32
 // accumulation):
-//   forward         one wavefront carries 16 contacts through all layers,
-//                   activations in LDS (16 x 128 BF16 per wave per buffer);
-//   backward        the same shape, dA = dZ W with W^T kept in HBM as BF16;
-//   weight gradient one 16 x 16 tile of dW per wavefront, the minibatch as
-//                   the MFMA reduction (activations and dZ are stored
-//                   feature-major so that both operands are contiguous);
-// then Adam on FP32 master weights and a BF16 re-cast of W and W^T.
+//   forward         four wavefronts carry 16 contacts through all layers, a
+//                   quarter of each layer's outputs a wave, activations in
+//                   LDS (16 x 128 BF16 per buffer);
+//   backward        goes on in the same workgroup from the pre-activations in
+//                   its registers, dA = dZ W with W^T kept in HBM as BF16;
+//   gradients       one launch: a wavefront per 16 x 16 tile of a dW, the
+//                   minibatch as the MFMA reduction (activations and dZ are
+//                   stored feature-major so that both operands are
+//                   contiguous), and a wavefront per bias;
+//   step            one launch: Adam on the FP32 master weights and the BF16
+//                   re-cast of W and W^T.
+// A minibatch of 1024 rows is 64 workgroups: the chip is mostly idle and a
+// step is the sum of its kernels' chains, so there are three of them.  As
+// sixteen launches (the rows' gather, a wave per 16 contacts, Z through HBM, a
+// launch per matrix) a step took 210 us; it takes ~50.
 //
 // MFMA 16x16x16 operand layout (wave64, lane l, i = 0..3):
 //   A (M x K):  lane holds A[l % 16][4 (l / 16) + i]
@@ -60,10 +68,11 @@ struct MlpWeights {
   const float* b[4];
 };
 
-// acc[t] = act x W^T for the 16 x 16 output tiles t = 0..NT-1, where act is
-// [16][K] (LDS) and W is [16 NT][K] (rows = outputs).
+// acc[t] = act x W^T for the 16 x 16 output tiles t0 .. t0 + NT - 1, where act
+// is [16][K] (LDS) and W is [rows = outputs][K].
 template <int K, int NT>
-__device__ __forceinline__ void wave_dense(const bf16* act, const bf16* __restrict__ W, f32x4* acc) {
+__device__ __forceinline__ void wave_dense(const bf16* act, const bf16* __restrict__ W, int t0,
+                                           f32x4* acc) {
   const int l = threadIdx.x & 63, row = l & 15, kq = l >> 4;
 #pragma unroll
   for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -73,7 +82,7 @@ __device__ __forceinline__ void wave_dense(const bf16* act, const bf16* __restri
 #pragma unroll
     for (int t = 0; t < NT; t++) {
       const bf16x4 b =
-          *reinterpret_cast<const bf16x4*>(&W[(size_t)(t * 16 + row) * K + k0 + 4 * kq]);
+          *reinterpret_cast<const bf16x4*>(&W[(size_t)((t0 + t) * 16 + row) * K + k0 + 4 * kq]);
       acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
     }
   }
@@ -81,160 +90,192 @@ __device__ __forceinline__ void wave_dense(const bf16* act, const bf16* __restri
 
 struct TrainBufs {
   int bsz;              // rows of the pass (multiple of 64)
-  float* Z[3];          // pre-activations [bsz][128]
   bf16* At[4];          // feature-major layer inputs: At[0] [32][bsz], At[l] [128][bsz]
-  float* out;           // [bsz][16]
   bf16* dZt[4];         // feature-major dZ: [128][bsz] for l = 0..2, [16][bsz] for l = 3
-  const float* target;  // [bsz][3]
-  float* loss_part;     // per-wave sum of squared errors
+  const int* idx;       // row r of the pass is row idx[r] of X and target; null: row r
+  const float* target;  // [rows][3]
+  float* loss_part;     // per 16 rows: sum of squared errors
 };
 
-// Forward pass, 16 contacts per wave, 4 waves per block; X is [>= 64 blocks][32]
-// standardised BF16 inputs.  Writes y[n][3] and, when training, what the
-// backward kernels need.
-template <bool TRAIN>
-__global__ __launch_bounds__(256) void k_mlp_forward(int n, const bf16* __restrict__ X,
-                                                     MlpWeights w, float* __restrict__ y,
-                                                     TrainBufs tb) {
-  __shared__ __attribute__((aligned(16))) bf16 buf[4][2][16 * MLP_H];
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int m0 = (blockIdx.x * 4 + wave) * 16;
-  bf16* a0 = buf[wave][0];
-  bf16* a1 = buf[wave][1];
-  for (int e = l; e < 16 * MLP_K1; e += 64) {
-    const int m = e / MLP_K1, k = e % MLP_K1;
-    const bf16 x = X[(size_t)(m0 + m) * MLP_K1 + k];
-    a0[m * MLP_K1 + k] = x;
-    if (TRAIN) tb.At[0][(size_t)k * tb.bsz + m0 + m] = x;
-  }
-  __syncthreads();
-  f32x4 acc[8];
-  const int col = l & 15, rq = l >> 4;
-  for (int layer = 0; layer < 3; layer++) {
-    const bf16* in = (layer & 1) ? a1 : a0;
-    bf16* outb = (layer & 1) ? a0 : a1;
-    if (layer == 0)
-      wave_dense<MLP_K1, 8>(in, w.w[0], acc);
-    else
-      wave_dense<MLP_H, 8>(in, w.w[layer], acc);
-    __syncthreads();
+// Four consecutive rows of one feature, feature-major (8-byte aligned: the
+// pass has a multiple of 64 rows).
+__device__ __forceinline__ void store4(bf16* p, const bf16* v) {
+  *reinterpret_cast<bf16x4*>(p) = bf16x4{(short)v[0], (short)v[1], (short)v[2], (short)v[3]};
+}
+
+// A hidden layer of the workgroup's 16 rows: this wave's two output tiles from
+// `in`, activations to `out`, pre-activations to z.
+template <int K>
+__device__ __forceinline__ void hidden_layer(const bf16* in, const bf16* __restrict__ W,
+                                             const float* __restrict__ b, int wave, bf16* out,
+                                             f32x4* z, bf16* At, int bsz, int m0) {
+  const int l = threadIdx.x & 63, col = l & 15, rq = l >> 4;
+  f32x4 acc[2];
+  wave_dense<K, 2>(in, W, 2 * wave, acc);
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
+  for (int t = 0; t < 2; t++) {
+    const int nn = (2 * wave + t) * 16 + col;
+    bf16 a[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int m = 4 * rq + i, nn = t * 16 + col;
-        const float z = acc[t][i] + w.b[layer][nn];
-        const bf16 a = f2bf(gelu(z));
-        outb[m * MLP_H + nn] = a;
-        if (TRAIN) {
-          tb.Z[layer][(size_t)(m0 + m) * MLP_H + nn] = z;
-          tb.At[layer + 1][(size_t)nn * tb.bsz + m0 + m] = a;
-        }
-      }
+    for (int i = 0; i < 4; i++) {
+      z[t][i] = acc[t][i] + b[nn];
+      a[i] = f2bf(gelu(z[t][i]));
+      out[(4 * rq + i) * MLP_H + nn] = a[i];
     }
-    __syncthreads();
+    if (At) store4(&At[(size_t)nn * bsz + m0 + 4 * rq], a);
   }
-  // output layer: the third hidden activation is in a1
-  wave_dense<MLP_H, 1>(a1, w.w[3], acc);
+}
+
+// Forward pass, 16 contacts per workgroup of 4 waves; X is [>= 16 blocks][32]
+// standardised BF16 inputs, y [n][3].
+__global__ __launch_bounds__(256) void k_mlp_forward(int n, const bf16* __restrict__ X,
+                                                     MlpWeights w, float* __restrict__ y) {
+  __shared__ __attribute__((aligned(16))) bf16 a0[16 * MLP_H], a1[16 * MLP_H];
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int m0 = blockIdx.x * 16;
+  for (int e = threadIdx.x; e < 16 * MLP_K1; e += 256) a0[e] = X[(size_t)m0 * MLP_K1 + e];
+  __syncthreads();
+  f32x4 z[2];
+  hidden_layer<MLP_K1>(a0, w.w[0], w.b[0], wave, a1, z, nullptr, 0, 0);
+  __syncthreads();
+  hidden_layer<MLP_H>(a1, w.w[1], w.b[1], wave, a0, z, nullptr, 0, 0);
+  __syncthreads();
+  hidden_layer<MLP_H>(a0, w.w[2], w.b[2], wave, a1, z, nullptr, 0, 0);
+  __syncthreads();
+  if (wave) return;
+  f32x4 acc[1];
+  wave_dense<MLP_H, 1>(a1, w.w[3], 0, acc);
+  const int col = l & 15, rq = l >> 4;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int m = 4 * rq + i;
     const float v = acc[0][i] + w.b[3][col];
     if (m0 + m < n && col < MLP_NO) y[(size_t)(m0 + m) * MLP_NO + col] = v;
-    if (TRAIN) tb.out[(size_t)(m0 + m) * MLP_NOP + col] = v;
   }
 }
 
-// Backward pass of the data path for the mean squared error over the first
-// `nvalid` rows: dZ of the output layer, then dA = dZ W and dZ = dA gelu'(Z)
-// down to the first layer, stored feature-major in BF16.
-__global__ __launch_bounds__(256) void k_mlp_backward(int nvalid, MlpWeights w, TrainBufs tb) {
-  __shared__ __attribute__((aligned(16))) bf16 buf[4][2][16 * MLP_H];
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int m0 = (blockIdx.x * 4 + wave) * 16;
-  const int col = l & 15, rq = l >> 4;
-  bf16* d0 = buf[wave][0];
-  bf16* d1 = buf[wave][1];
-  const float scale = 2.0f / (float)(nvalid * MLP_NO);
-  float lsum = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int m = 4 * rq + i;
-    float g = 0.f;
-    if (col < MLP_NO && m0 + m < nvalid) {
-      const float diff = tb.out[(size_t)(m0 + m) * MLP_NOP + col] -
-                         tb.target[(size_t)(m0 + m) * MLP_NO + col];
-      g = scale * diff;
-      lsum += diff * diff;
-    }
-    const bf16 gb = f2bf(g);
-    d0[m * MLP_NOP + col] = gb;
-    tb.dZt[3][(size_t)col * tb.bsz + m0 + m] = gb;
+// Forward and backward of the data path for the mean squared error over the
+// first `nvalid` rows, 16 rows per workgroup: dZ of the output layer, then dA =
+// dZ W and dZ = dA gelu'(Z) down to the first layer.  Layer inputs and dZ go
+// out feature-major in BF16.
+__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(int nvalid, const bf16* __restrict__ X,
+                                                     MlpWeights w, TrainBufs tb) {
+  __shared__ __attribute__((aligned(16))) bf16 a0[16 * MLP_H], a1[16 * MLP_H], d3[16 * MLP_NOP];
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, col = l & 15, rq = l >> 4;
+  const int m0 = blockIdx.x * 16;
+  for (int e = threadIdx.x; e < 16 * MLP_K1; e += 256) {
+    const int m = e / MLP_K1, k = e % MLP_K1;
+    const int src = tb.idx ? tb.idx[m0 + m] : m0 + m;
+    const bf16 x = X[(size_t)src * MLP_K1 + k];
+    a0[e] = x;
+    tb.At[0][(size_t)k * tb.bsz + m0 + m] = x;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
-  if (l == 0) tb.loss_part[blockIdx.x * 4 + wave] = lsum;
   __syncthreads();
-  f32x4 acc[8];
-  // dA of the third hidden layer = dZ4 W4 (reduction over the 16 outputs)
-  wave_dense<MLP_NOP, 8>(d0, w.wt[3], acc);
+  f32x4 z0[2], z1[2], z2[2], acc[2];
+  hidden_layer<MLP_K1>(a0, w.w[0], w.b[0], wave, a1, z0, tb.At[1], tb.bsz, m0);
   __syncthreads();
-  bf16* cur = d1;
-  for (int layer = 2; layer >= 0; layer--) {
+  hidden_layer<MLP_H>(a1, w.w[1], w.b[1], wave, a0, z1, tb.At[2], tb.bsz, m0);
+  __syncthreads();
+  hidden_layer<MLP_H>(a0, w.w[2], w.b[2], wave, a1, z2, tb.At[3], tb.bsz, m0);
+  __syncthreads();
+  if (wave == 0) {
+    wave_dense<MLP_H, 1>(a1, w.w[3], 0, acc);
+    const float scale = 2.0f / (float)(nvalid * MLP_NO);
+    float lsum = 0.f;
+    bf16 gb[4];
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
+    for (int i = 0; i < 4; i++) {
+      const int m = 4 * rq + i;
+      const float v = acc[0][i] + w.b[3][col];
+      float g = 0.f;
+      if (col < MLP_NO && m0 + m < nvalid) {
+        const int src = tb.idx ? tb.idx[m0 + m] : m0 + m;
+        const float diff = v - tb.target[(size_t)src * MLP_NO + col];
+        g = scale * diff;
+        lsum += diff * diff;
+      }
+      gb[i] = f2bf(g);
+      d3[m * MLP_NOP + col] = gb[i];
+    }
+    store4(&tb.dZt[3][(size_t)col * tb.bsz + m0 + 4 * rq], gb);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
+    if (l == 0) tb.loss_part[blockIdx.x] = lsum;
+  }
+  __syncthreads();
+  // dZ of a layer from dA (acc) and its pre-activations
+  auto dz = [&](const f32x4* z, bf16* out, bf16* dZt) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int nn = (2 * wave + t) * 16 + col;
+      bf16 g[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int m = 4 * rq + i, nn = t * 16 + col;
-        const float z = tb.Z[layer][(size_t)(m0 + m) * MLP_H + nn];
-        const bf16 g = f2bf(acc[t][i] * gelu_grad(z));
-        cur[m * MLP_H + nn] = g;
-        tb.dZt[layer][(size_t)nn * tb.bsz + m0 + m] = g;
+        g[i] = f2bf(acc[t][i] * gelu_grad(z[t][i]));
+        if (out) out[(4 * rq + i) * MLP_H + nn] = g[i];
       }
+      store4(&dZt[(size_t)nn * tb.bsz + m0 + 4 * rq], g);
     }
-    __syncthreads();
-    if (layer == 0) break;
-    // dA of layer `layer - 1`'s output = dZ_layer W_layer
-    wave_dense<MLP_H, 8>(cur, w.wt[layer], acc);
-    __syncthreads();
-    cur = (cur == d1) ? d0 : d1;
-  }
+  };
+  // dA of the third hidden layer = dZ4 W4 (reduction over the 16 outputs)
+  wave_dense<MLP_NOP, 2>(d3, w.wt[3], 2 * wave, acc);
+  dz(z2, a0, tb.dZt[2]);
+  __syncthreads();
+  wave_dense<MLP_H, 2>(a0, w.wt[2], 2 * wave, acc);
+  dz(z1, a1, tb.dZt[1]);
+  __syncthreads();
+  wave_dense<MLP_H, 2>(a1, w.wt[1], 2 * wave, acc);
+  dz(z0, nullptr, tb.dZt[0]);
 }
 
-// dW[n][k] = sum_m dZ[m][n] A[m][k]: one 16 x 16 tile per wave.
-__global__ __launch_bounds__(256) void k_mlp_wgrad(int bsz, const bf16* __restrict__ dZt,
-                                                   const bf16* __restrict__ At, int kin,
-                                                   float* __restrict__ dW, int ntiles) {
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int tile = blockIdx.x * 4 + wave;
-  if (tile >= ntiles) return;
-  const int ktiles = kin / 16;
-  const int n0 = (tile / ktiles) * 16, k0 = (tile % ktiles) * 16;
-  const int r = l & 15, q = l >> 4;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int m0 = 0; m0 < bsz; m0 += 16) {
-    const bf16x4 a = *reinterpret_cast<const bf16x4*>(&dZt[(size_t)(n0 + r) * bsz + m0 + 4 * q]);
-    const bf16x4 b = *reinterpret_cast<const bf16x4*>(&At[(size_t)(k0 + r) * bsz + m0 + 4 * q]);
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-  }
+// All gradients: dW[n][k] = sum_m dZ[m][n] A[m][k], one 16 x 16 tile per wave
+// (the loads of eight steps in flight), then db[n] = sum_m dZ[m][n], one wave
+// per output with fixed-order lane sums.
+constexpr int MLP_TILES[4] = {(MLP_H / 16) * (MLP_K1 / 16), (MLP_H / 16) * (MLP_H / 16),
+                              (MLP_H / 16) * (MLP_H / 16), (MLP_NOP / 16) * (MLP_H / 16)};
+constexpr int MLP_ALL_TILES = MLP_TILES[0] + MLP_TILES[1] + MLP_TILES[2] + MLP_TILES[3];
+constexpr int MLP_GRAD_WAVES = MLP_ALL_TILES + 3 * MLP_H + MLP_NOP;
+__global__ __launch_bounds__(256) void k_mlp_grads(TrainBufs tb, float* __restrict__ grads) {
+  const int l = threadIdx.x & 63, bsz = tb.bsz;
+  int wv = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (wv >= MLP_GRAD_WAVES) return;
+  constexpr int woff[4] = {OW1, OW2, OW3, OW4}, boff[4] = {OB1, OB2, OB3, OB4};
+  if (wv < MLP_ALL_TILES) {
+    int layer = 0;
+    while (wv >= MLP_TILES[layer]) wv -= MLP_TILES[layer++];
+    const int kin = layer == 0 ? MLP_K1 : MLP_H, ktiles = kin / 16;
+    const int n0 = (wv / ktiles) * 16, k0 = (wv % ktiles) * 16;
+    const int r = l & 15, q = l >> 4;
+    const bf16* __restrict__ pa = tb.dZt[layer] + (size_t)(n0 + r) * bsz + 4 * q;
+    const bf16* __restrict__ pb = tb.At[layer] + (size_t)(k0 + r) * bsz + 4 * q;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int m0 = 0; m0 < bsz; m0 += 16) {
+      const bf16x4 a = *reinterpret_cast<const bf16x4*>(pa + m0);
+      const bf16x4 b = *reinterpret_cast<const bf16x4*>(pb + m0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    }
+    float* dW = grads + woff[layer];
 #pragma unroll
-  for (int i = 0; i < 4; i++) dW[(size_t)(n0 + 4 * q + i) * kin + k0 + r] = acc[i];
-}
-
-// db[n] = sum_m dZ[m][n], one wave per output, fixed-order lane sums
-__global__ __launch_bounds__(64) void k_mlp_bgrad(int bsz, const bf16* __restrict__ dZt,
-                                                  float* __restrict__ db) {
-  const int nn = blockIdx.x, l = threadIdx.x;
+    for (int i = 0; i < 4; i++) dW[(size_t)(n0 + 4 * q + i) * kin + k0 + r] = acc[i];
+    return;
+  }
+  wv -= MLP_ALL_TILES;
+  const int layer = wv / MLP_H, nn = wv % MLP_H;  // (the last layer has 16 outputs)
+  const bf16* __restrict__ d = tb.dZt[layer] + (size_t)nn * bsz;
   float s = 0.f;
-  for (int m = l; m < bsz; m += 64) s += bf2f(dZt[(size_t)nn * bsz + m]);
+#pragma unroll 8
+  for (int m = l; m < bsz; m += 64) s += bf2f(d[m]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if (l == 0) db[nn] = s;
+  if (l == 0) grads[boff[layer] + nn] = s;
 }
 
+// Adam, and the BF16 copies of the weight it moved ([n][k] and [k][n]).
 __global__ void k_adam(int np, float* __restrict__ p, const float* __restrict__ g,
                        float* __restrict__ m1, float* __restrict__ m2, float lr, float b1, float b2,
-                       float c1, float c2, float eps) {
+                       float c1, float c2, float eps, bf16* w0, bf16* wt0, bf16* w1, bf16* wt1,
+                       bf16* w2, bf16* wt2, bf16* w3, bf16* wt3) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
   const float gi = g[i];
@@ -242,7 +283,19 @@ __global__ void k_adam(int np, float* __restrict__ p, const float* __restrict__ 
   const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
   m1[i] = a;
   m2[i] = b;
-  p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+  const float v = p[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
+  p[i] = v;
+  auto cast = [&](int off, int nout, int kin, bf16* w, bf16* wt) {
+    const int e = i - off;
+    if (e < 0 || e >= nout * kin) return;
+    const bf16 x = f2bf(v);
+    w[e] = x;
+    wt[(size_t)(e % kin) * nout + e / kin] = x;
+  };
+  cast(OW1, MLP_H, MLP_K1, w0, wt0);
+  cast(OW2, MLP_H, MLP_H, w1, wt1);
+  cast(OW3, MLP_H, MLP_H, w2, wt2);
+  cast(OW4, MLP_NOP, MLP_H, w3, wt3);
 }
 
 // BF16 copies of one weight matrix, [n][k] and transposed [k][n]
@@ -266,18 +319,6 @@ __global__ void k_mlp_inputs(int n, int npad, const float* __restrict__ f,
   X[i] = (k < MLP_NF && m < n) ? f2bf((f[(size_t)m * MLP_NF + k] - mean[k]) / stdv[k]) : (bf16)0;
 }
 
-// minibatch rows: bx[r] = X[idx[r]], bt[r] = T[idx[r]]
-__global__ void k_mlp_gather(int batch, const int* __restrict__ idx, const bf16* __restrict__ X,
-                             const float* __restrict__ T, bf16* __restrict__ bx,
-                             float* __restrict__ bt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= batch * MLP_K1) return;
-  const int r = i / MLP_K1, k = i % MLP_K1;
-  const int src = idx[r];
-  bx[i] = X[(size_t)src * MLP_K1 + k];
-  if (k < MLP_NO) bt[(size_t)r * MLP_NO + k] = T[(size_t)src * MLP_NO + k];
-}
-
 }  // namespace fc3d
 
 using namespace fc3d;
@@ -292,10 +333,9 @@ struct fc3d_hip_mlp {
   long adam_t = 0;
   // training workspace for passes of up to ws_bsz rows
   int ws_bsz = 0;
-  float* Z[3] = {nullptr, nullptr, nullptr};
   bf16* At[4] = {nullptr, nullptr, nullptr, nullptr};
   bf16* dZt[4] = {nullptr, nullptr, nullptr, nullptr};
-  float *out = nullptr, *loss_part = nullptr;
+  float* loss_part = nullptr;
 };
 
 namespace fc3d {
@@ -315,12 +355,6 @@ static MlpWeights mlp_weights(const fc3d_hip_mlp* m) {
   return w;
 }
 
-static TrainBufs no_train() {
-  TrainBufs t;
-  std::memset(&t, 0, sizeof t);
-  return t;
-}
-
 static int mlp_cast(fc3d_hip_mlp* m) {
   for (int k = 0; k < 4; k++) {
     const int n = kDims[k][0] * kDims[k][1];
@@ -332,18 +366,13 @@ static int mlp_cast(fc3d_hip_mlp* m) {
 }
 
 static void free_workspace(fc3d_hip_mlp* m) {
-  for (int k = 0; k < 3; k++) {
-    hipFree(m->Z[k]);
-    m->Z[k] = nullptr;
-  }
   for (int k = 0; k < 4; k++) {
     hipFree(m->At[k]);
     hipFree(m->dZt[k]);
     m->At[k] = m->dZt[k] = nullptr;
   }
-  hipFree(m->out);
   hipFree(m->loss_part);
-  m->out = m->loss_part = nullptr;
+  m->loss_part = nullptr;
   m->ws_bsz = 0;
 }
 
@@ -351,43 +380,33 @@ static int mlp_workspace(fc3d_hip_mlp* m, int bsz) {
   if (m->ws_bsz >= bsz) return 0;
   FC3D_HIP_TRY(hipStreamSynchronize(m->stream));
   free_workspace(m);
-  for (int k = 0; k < 3; k++) FC3D_HIP_TRY(hipMalloc(&m->Z[k], sizeof(float) * bsz * MLP_H));
   FC3D_HIP_TRY(hipMalloc(&m->At[0], sizeof(bf16) * bsz * MLP_K1));
   for (int k = 1; k < 4; k++) FC3D_HIP_TRY(hipMalloc(&m->At[k], sizeof(bf16) * bsz * MLP_H));
   for (int k = 0; k < 3; k++) FC3D_HIP_TRY(hipMalloc(&m->dZt[k], sizeof(bf16) * bsz * MLP_H));
   FC3D_HIP_TRY(hipMalloc(&m->dZt[3], sizeof(bf16) * bsz * MLP_NOP));
-  FC3D_HIP_TRY(hipMalloc(&m->out, sizeof(float) * bsz * MLP_NOP));
   FC3D_HIP_TRY(hipMalloc(&m->loss_part, sizeof(float) * (bsz / 16)));
   m->ws_bsz = bsz;
   return 0;
 }
 
-// Forward + backward over `bsz` rows (the first `nvalid` carry targets):
-// gradients into m->g, per-wave loss partials into m->loss_part.
-static int mlp_grad_pass(fc3d_hip_mlp* m, int nvalid, int bsz, const bf16* X, const float* T) {
+// Forward + backward over `bsz` rows (the first `nvalid` carry targets; idx
+// picks them from X and T, null: the rows in order): gradients into m->g, loss
+// partials into m->loss_part.
+static int mlp_grad_pass(fc3d_hip_mlp* m, int nvalid, int bsz, const bf16* X, const float* T,
+                         const int* idx) {
   TrainBufs tb;
   tb.bsz = bsz;
-  for (int k = 0; k < 3; k++) tb.Z[k] = m->Z[k];
   for (int k = 0; k < 4; k++) {
     tb.At[k] = m->At[k];
     tb.dZt[k] = m->dZt[k];
   }
-  tb.out = m->out;
+  tb.idx = idx;
   tb.target = T;
   tb.loss_part = m->loss_part;
-  const MlpWeights w = mlp_weights(m);
-  const int blocks = bsz / 64;
-  hipLaunchKernelGGL(k_mlp_forward<true>, dim3(blocks), dim3(256), 0, m->stream, 0, X, w,
-                     (float*)nullptr, tb);
-  hipLaunchKernelGGL(k_mlp_backward, dim3(blocks), dim3(256), 0, m->stream, nvalid, w, tb);
-  for (int k = 0; k < 4; k++) {
-    const int nout = kDims[k][0], kin = kDims[k][1];
-    const int ntiles = (nout / 16) * (kin / 16);
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3((ntiles + 3) / 4), dim3(256), 0, m->stream, bsz,
-                       m->dZt[k], m->At[k], kin, m->g + kWOff[k], ntiles);
-    hipLaunchKernelGGL(k_mlp_bgrad, dim3(nout), dim3(64), 0, m->stream, bsz, m->dZt[k],
-                       m->g + kBOff[k]);
-  }
+  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(bsz / 16), dim3(256), 0, m->stream, nvalid, X,
+                     mlp_weights(m), tb);
+  hipLaunchKernelGGL(k_mlp_grads, dim3((MLP_GRAD_WAVES + 3) / 4), dim3(256), 0, m->stream, tb,
+                     m->g);
   FC3D_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -414,8 +433,7 @@ int mlp_forward_device(fc3d_hip_mlp* m, int n, const float* feat, bf16* X, float
   const int npad = (n + 63) / 64 * 64;
   hipLaunchKernelGGL(k_mlp_inputs, dim3((unsigned)(((size_t)npad * MLP_K1 + 255) / 256)),
                      dim3(256), 0, s, n, npad, feat, m->mean, m->stdv, X);
-  hipLaunchKernelGGL(k_mlp_forward<false>, dim3(npad / 64), dim3(256), 0, s, n, X,
-                     mlp_weights(m), y, no_train());
+  hipLaunchKernelGGL(k_mlp_forward, dim3(npad / 16), dim3(256), 0, s, n, X, mlp_weights(m), y);
   FC3D_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -591,7 +609,7 @@ int fc3d_hip_mlp_gradients(fc3d_hip_mlp* m, int n, const float* x, const float* 
                               m->stream));
   hipLaunchKernelGGL(k_mlp_inputs, dim3((unsigned)(((size_t)bsz * MLP_K1 + 255) / 256)),
                      dim3(256), 0, m->stream, n, bsz, df, m->mean, m->stdv, dx);
-  if ((rc = mlp_grad_pass(m, n, bsz, dx, dt))) return rc;
+  if ((rc = mlp_grad_pass(m, n, bsz, dx, dt, nullptr))) return rc;
   const double s = sum_loss(m, bsz, &rc);
   if (rc) return rc;
   if (grads) FC3D_HIP_TRY(hipMemcpy(grads, m->g, sizeof(float) * NPARAM, hipMemcpyDeviceToHost));
@@ -630,15 +648,13 @@ int fc3d_hip_mlp_train(fc3d_hip_mlp* m, int n, const float* x, const float* t, i
   }
   if ((rc = mlp_workspace(m, batch))) return rc;
   DevBufs B;
-  float *df = nullptr, *dt = nullptr, *bt = nullptr;
-  bf16 *dx = nullptr, *bx = nullptr;
+  float *df = nullptr, *dt = nullptr;
+  bf16* dx = nullptr;
   int* didx = nullptr;
   const int steps = std::max(1, n / batch);
   FC3D_HIP_TRY(B.get(&df, (size_t)n * MLP_NF));
   FC3D_HIP_TRY(B.get(&dx, (size_t)n * MLP_K1));
   FC3D_HIP_TRY(B.get(&dt, (size_t)n * MLP_NO));
-  FC3D_HIP_TRY(B.get(&bx, (size_t)batch * MLP_K1));
-  FC3D_HIP_TRY(B.get(&bt, (size_t)batch * MLP_NO));
   FC3D_HIP_TRY(B.get(&didx, (size_t)steps * batch));
   FC3D_HIP_TRY(hipMemcpyAsync(df, x, sizeof(float) * (size_t)n * MLP_NF, hipMemcpyHostToDevice,
                               m->stream));
@@ -657,15 +673,14 @@ int fc3d_hip_mlp_train(fc3d_hip_mlp* m, int n, const float* x, const float* t, i
     // the stream is idle here (previous epoch ended with a synchronize)
     FC3D_HIP_TRY(hipMemcpy(didx, idx.data(), sizeof(int) * idx.size(), hipMemcpyHostToDevice));
     for (int s = 0; s < steps; s++) {
-      hipLaunchKernelGGL(k_mlp_gather, dim3((batch * MLP_K1 + 255) / 256), dim3(256), 0,
-                         m->stream, batch, didx + (size_t)s * batch, dx, dt, bx, bt);
-      if ((rc = mlp_grad_pass(m, batch, batch, bx, bt))) return rc;
+      if ((rc = mlp_grad_pass(m, batch, batch, dx, dt, didx + (size_t)s * batch))) return rc;
       m->adam_t++;
       const float c1 = 1.f - (float)std::pow((double)b1, (double)m->adam_t);
       const float c2 = 1.f - (float)std::pow((double)b2, (double)m->adam_t);
       hipLaunchKernelGGL(k_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, m->stream, NPARAM,
-                         m->p, m->g, m->m1, m->m2, lr, b1, b2, c1, c2, 1e-8f);
-      if ((rc = mlp_cast(m))) return rc;
+                         m->p, m->g, m->m1, m->m2, lr, b1, b2, c1, c2, 1e-8f, m->w[0], m->wt[0],
+                         m->w[1], m->wt[1], m->w[2], m->wt[2], m->w[3], m->wt[3]);
+      FC3D_HIP_TRY(hipGetLastError());
     }
     // the last minibatch's loss was computed with the weights before its step
     last = sum_loss(m, batch, &rc) / ((double)batch * MLP_NO);
