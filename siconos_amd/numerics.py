@@ -39,6 +39,28 @@ NUMERICS_ERR_MAX_ITER = -20
 _libc = C.CDLL(None)
 _libc.malloc.restype = C.c_void_p
 _libc.malloc.argtypes = [C.c_size_t]
+_libc.free.restype = None
+_libc.free.argtypes = [C.c_void_p]
+
+
+class _Owned:
+    """A malloc'ed C array handed to numpy without a copy: the arrays made from
+    it keep this object alive, which frees the memory."""
+
+    def __init__(self, address, n, typestr):
+        self._p = address
+        self.__array_interface__ = {"shape": (n,), "typestr": typestr, "version": 3,
+                                    "data": (self._p, False)}
+
+    def __del__(self):
+        _libc.free(self._p)
+
+
+def _take(g, field, n, typestr):
+    """Field of a fc3d_generated as an array that owns its memory."""
+    address = C.cast(getattr(g, field), C.c_void_p).value
+    setattr(g, field, None)
+    return np.asarray(_Owned(address, n, typestr))
 
 
 def dptr(a):
@@ -407,10 +429,9 @@ def assemble(nbodies, body_a, body_b, H, minv, vfree, minv_diagonal=True, device
         raise RuntimeError(f"fc3d_hip_assemble: {rc} {capi.last_error()}")
     try:
         nb = g.nnzb
-        W = SparseBlock3(np.ctypeslib.as_array(g.row_ptr, shape=(nc + 1,)).copy(),
-                         np.ctypeslib.as_array(g.col_idx, shape=(nb,)).copy(),
-                         np.ctypeslib.as_array(g.blocks, shape=(nb * 9,)).copy())
-        q = np.ctypeslib.as_array(g.q, shape=(3 * nc,)).copy()
+        W = SparseBlock3(_take(g, "row_ptr", nc + 1, "<i8"), _take(g, "col_idx", nb, "<i8"),
+                         _take(g, "blocks", nb * 9, "<f8"))
+        q = _take(g, "q", 3 * nc, "<f8")
     finally:
         lib.fc3d_generated_free(C.byref(g))
     return W, q, ms.value

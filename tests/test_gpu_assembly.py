@@ -115,3 +115,37 @@ def test_assembly_of_blocks_with_several_shared_sides(lib, diagonal):
     # the case mix the test is for
     pairs = lambda c, d: sum(1 for x in (ba[c], bb[c]) for y in (ba[d], bb[d]) if x >= 0 and x == y)
     assert pairs(0, 40) == 2 and pairs(10, 50) == 2 and pairs(55, 55) == 4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nc", [100, 32768, 50001])
+def test_structure_by_row_ranges(nc):
+    """The block structure below and above the size that is built by several
+    threads, with contacts of one body, of none and of the same body twice,
+    against a row-by-row construction; the arrays stay valid after every other
+    reference to the call is gone."""
+    import gc
+    rng = np.random.default_rng(nc)
+    nb = nc // 3 + 2
+    a = rng.integers(0, nb, nc).astype(np.int32)
+    b = rng.integers(0, nb, nc).astype(np.int32)
+    a[::17], b[::23], b[::29] = -1, -1, a[::29]
+    H, minv, v = rng.normal(size=36 * nc), rng.uniform(0.5, 2.0, 6 * nb), rng.normal(size=6 * nb)
+    W, q, _ = N.assemble(nb, a, b, H, minv, v)
+    gc.collect()
+    at = [[] for _ in range(nb)]
+    for c in range(nc):
+        for k in {int(a[c]), int(b[c])} - {-1}:
+            at[k].append(c)
+    for c in range(nc):
+        want = {c}
+        for k in (a[c], b[c]):
+            if k >= 0:
+                want |= set(at[k])
+        np.testing.assert_array_equal(W.col_idx[W.row_ptr[c]:W.row_ptr[c + 1]], sorted(want))
+    c = nc // 2
+    h = H[36 * c:36 * c + 36].reshape(12, 3)
+    u = sum((h[6 * s:6 * s + 6].T @ v[6 * k:6 * k + 6] for s, k in enumerate((a[c], b[c]))
+             if k >= 0), np.zeros(3))
+    np.testing.assert_allclose(q[3 * c:3 * c + 3], u, rtol=1e-12, atol=1e-12)
+    assert W.values.flags.writeable and W.values.shape == (W.row_ptr[-1], 9)
