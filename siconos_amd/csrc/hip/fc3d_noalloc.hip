@@ -54,17 +54,26 @@ __device__ __forceinline__ void add_block(const double* w, const double* __restr
   mvp3x3<double>(w, v, u);
 }
 
-// One wave per 64 contacts.  Their rows are one range of the CSR, which the
-// wave walks CSR_CHUNK blocks at a time: coalesced 512-byte loads of the
+// WPR waves per 64 contacts.  Their rows are one range of the CSR, which the
+// waves walk CSR_CHUNK blocks a wave at a time: coalesced 512-byte loads of the
 // blocks into LDS, a lane per block for its products with the neighbour's
-// reaction (every gather of a chunk in flight), then a lane per row adds its
-// row's products in their order.  HBM bounds it (0.85 GB for 1M contacts with
-// 10.5M blocks): 1.8 TB/s when a lane walked its own row, 72 bytes in another
-// 128-byte line than its neighbours at every step (483 us a call, both
-// kernels), 4.1 TB/s so (208 us; a copy reaches 5.1).  A wave with a bad row
-// walks its rows from memory: every form of row pointers that was accepted
-// still is.
+// reaction (every gather of a chunk in flight), then a lane of the first wave
+// per row adds its row's products in their order.  HBM bounds a large problem
+// (0.85 GB for 1M contacts with 10.5M blocks): 1.8 TB/s when a lane walked its
+// own row, 72 bytes in another 128-byte line than its neighbours at every step
+// (480 us a call, both kernels), 4.1 TB/s so (207 us; a copy reaches 5.1).  A
+// wave with a bad row walks its rows from memory: every form of row pointers
+// that was accepted still is.
+//
+// A problem that leaves the GPU's wave slots empty is bound by the chain of a
+// wave's chunks, and four waves per 64 contacts walk a quarter of it each; a
+// larger one has the waves, and gains by not waiting for each other.  us a call
+// (a lane per row / one wave / four waves): 1000 contacts 15.4 / 24.4 / 11.7,
+// 16k 16.3 / 24.9 / 12.0, 64k 28.1 / 27.5 / 22.6, 256k 122 / 61.7 / 55.2, 512k
+// 249 / 111 / 119, 1M 480 / 207 / 226.
 constexpr int CSR_CHUNK = 128;
+constexpr int CSR_WIDE_CONTACTS = 1 << 18;
+template <int WPR>
 __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
                                                       const int64_t* __restrict__ rp,
                                                       const int64_t* __restrict__ ci,
@@ -74,9 +83,18 @@ __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
                                                       const double* __restrict__ r,
                                                       double* __restrict__ u_out,
                                                       double* __restrict__ part) {
-  __shared__ double sblk[4][CSR_CHUNK * 9];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  constexpr int T = 64 * WPR, CHUNK = CSR_CHUNK * WPR, G = 4 / WPR;
+  __shared__ double sblk[G][CHUNK * 9];
+  const int group = threadIdx.x / T, t = threadIdx.x % T, lane = threadIdx.x & 63;
+  const int i = (blockIdx.x * G + group) * 64 + lane;
+  auto sync = [] {
+    if constexpr (WPR == 1) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      __syncthreads();  // G = 1: the block's waves hold the same rows and walk the same chunks
+    }
+  };
   double e2 = 0.0, r2 = 0.0, u2 = 0.0;
   double u[3] = {0.0, 0.0, 0.0};
   int64_t k0 = 0, k1 = 0;
@@ -94,17 +112,17 @@ __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
   const int64_t kb = __shfl(k0, 0, 64), ke = last >= 0 ? __shfl(k1, last, 64) : 0;
   if (plain && last >= 0) {
     int64_t k = k0;
-    for (int64_t c0 = kb; c0 < ke; c0 += CSR_CHUNK) {
-      const int n = (int)min((int64_t)CSR_CHUNK, ke - c0);
+    for (int64_t c0 = kb; c0 < ke; c0 += CHUNK) {
+      const int n = (int)min((int64_t)CHUNK, ke - c0);
       const double* __restrict__ src = blocks + 9 * c0;
-      double t[CSR_CHUNK * 9 / 64], v[CSR_CHUNK / 64][3];
+      double b9[CSR_CHUNK * 9 / 64], v[CSR_CHUNK / 64][3];
       int64_t jc[CSR_CHUNK / 64];
 #pragma unroll
       for (int x = 0; x < CSR_CHUNK / 64; x++)
-        jc[x] = x * 64 + lane < n ? ci[c0 + x * 64 + lane] : 0;
+        jc[x] = x * T + t < n ? ci[c0 + x * T + t] : 0;
 #pragma unroll
       for (int x = 0; x < CSR_CHUNK * 9 / 64; x++)
-        if (x * 64 + lane < 9 * n) t[x] = src[x * 64 + lane];
+        if (x * T + t < 9 * n) b9[x] = src[x * T + t];
 #pragma unroll
       for (int x = 0; x < CSR_CHUNK / 64; x++) {
         const bool ok = jc[x] >= 0 && jc[x] < nc;
@@ -116,28 +134,25 @@ __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
       }
 #pragma unroll
       for (int x = 0; x < CSR_CHUNK * 9 / 64; x++)
-        if (x * 64 + lane < 9 * n) sblk[wave][x * 64 + lane] = t[x];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+        if (x * T + t < 9 * n) sblk[group][x * T + t] = b9[x];
+      sync();
 #pragma unroll
       for (int x = 0; x < CSR_CHUNK / 64; x++)
-        if (x * 64 + lane < n) {
-          double* b = &sblk[wave][9 * (x * 64 + lane)];
+        if (x * T + t < n) {
+          double* b = &sblk[group][9 * (x * T + t)];
 #pragma unroll
           for (int e = 0; e < 9; e++) b[e] = b[e] * v[x][e / 3];
         }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      sync();
       // u += W r_j as mvp3x3 adds it: column after column
-      for (const int64_t stop = min(k1, c0 + n); k < stop; k++) {
-        const double* b = &sblk[wave][9 * (int)(k - c0)];
+      for (const int64_t stop = WPR == 1 || t < 64 ? min(k1, c0 + n) : k; k < stop; k++) {
+        const double* b = &sblk[group][9 * (int)(k - c0)];
 #pragma unroll
         for (int e = 0; e < 9; e++) u[e % 3] += b[e];
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();  // the chunk is read before the next one lands
+      sync();  // the chunk is read before the next one lands
     }
-  } else if (i < nc) {
+  } else if (i < nc && t < 64) {
     for (int64_t k = bad ? k1 : k0; k < k1; k++) {
       const int64_t j = ci[k];
       if (j < 0 || j >= nc) {
@@ -150,6 +165,7 @@ __global__ __launch_bounds__(256) void k_csr_residual(int nc, int64_t nnzb,
       add_block(w, r, j, u);
     }
   }
+  if (t >= 64) return;  // the first wave has the rows
   if (i < nc) {
     if (bad) u[0] = u[1] = u[2] = NAN;
 #pragma unroll
@@ -220,8 +236,10 @@ int fc3d_hip_compute_error_device(int nc, int64_t nnzb, const int64_t* row_ptr,
   if ((rc = scratch_on(device, &part))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int nwaves = (nc + 63) / 64;
-  hipLaunchKernelGGL(k_csr_residual, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, nc,
-                     nnzb, row_ptr, col_idx, blocks, q, mu, reaction, velocity, part);
+  const bool wide = nc <= CSR_WIDE_CONTACTS;
+  hipLaunchKernelGGL(wide ? k_csr_residual<4> : k_csr_residual<1>,
+                     dim3((unsigned)(wide ? nwaves : (nwaves + 3) / 4)), dim3(256), 0, s, nc, nnzb,
+                     row_ptr, col_idx, blocks, q, mu, reaction, velocity, part);
   hipLaunchKernelGGL(k_csr_residual_end, dim3(1), dim3(1024), 0, s, (const double*)part, nwaves,
                      norm, error);
   FC3D_HIP_TRY(hipGetLastError());

@@ -6,6 +6,7 @@
 // a host loop over a downloaded copy of the slots it took ~9 ms for each
 // vector of 1M contacts, an eighth of the fast method's solve.)
 #pragma once
+#include <mutex>
 #include <vector>
 
 #include "fc3d_internal.hpp"
@@ -37,12 +38,15 @@ static __global__ void k_contacts_to_slots(int nslots, const int* __restrict__ s
                                   in[3 * (size_t)i + 2], 0.0);
 }
 
-// Device side of a handle's transfers, allocated on first use.
+// Device side of a handle's transfers, allocated on first use.  Threads that
+// read one handle at the same time take turns with its buffer.
 struct Transfer {
+  std::mutex turn;
   int *o2s = nullptr, *s2o = nullptr;
   double* buf = nullptr;  // three values a contact
 
   int ensure(const std::vector<int>& orig2slot, const std::vector<int>& slot2orig) {
+    std::lock_guard<std::mutex> lock(turn);
     if (buf) return 0;
     const size_t n = orig2slot.size(), ns = slot2orig.size();
     if (!o2s) FC3D_HIP_TRY(hipMalloc(&o2s, sizeof(int) * n));
@@ -53,6 +57,7 @@ struct Transfer {
     return 0;
   }
   int to_host(int n, const double4* slots, double* out, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(turn);
     hipLaunchKernelGGL(k_slots_to_contacts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n,
                        (const int*)o2s, slots, buf);
     FC3D_HIP_TRY(hipGetLastError());
@@ -62,6 +67,7 @@ struct Transfer {
     return 0;
   }
   int to_device(int n, int nslots, const double* in, double4* slots, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(turn);
     FC3D_HIP_TRY(hipMemcpyAsync(buf, in, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice,
                                 s));
     hipLaunchKernelGGL(k_contacts_to_slots, dim3((unsigned)((nslots + 255) / 256)), dim3(256), 0,

@@ -134,3 +134,34 @@ def test_no_alloc_residual_rows_of_every_length(nc):
         type(short).nnzb = property(lambda s: int(s.row_ptr[-1]))
     assert rc == 0 and np.isnan(err) and np.isnan(u[-3:]).all()
     np.testing.assert_array_equal(u[:-3], want.reshape(-1)[:-3])
+
+
+@pytest.mark.parametrize("nc", [262144, 262209])
+def test_no_alloc_residual_on_both_sides_of_its_wide_form(nc):
+    """The largest problem that takes four waves per 64 contacts and one that
+    takes one wave, its last wave ragged: rows of 0 to 7 blocks and one of 300,
+    then a column out of range."""
+    rng = np.random.default_rng(nc)
+    per = rng.integers(0, 8, nc)
+    per[nc - 70] = 300
+    rp = np.concatenate([[0], np.cumsum(per)])
+    ci = rng.integers(0, nc, rp[-1])
+    blocks = rng.normal(size=(rp[-1], 9))
+    q, r = rng.normal(size=3 * nc), rng.normal(size=3 * nc)
+    want = q.copy().reshape(-1, 3)
+    for k in range(300):
+        rows = np.flatnonzero(per > k)
+        b = blocks[rp[rows] + k]
+        x = r.reshape(-1, 3)[ci[rp[rows] + k]]
+        for j in range(3):  # column after column, as mvp3x3
+            want[rows] += b[:, 3 * j:3 * j + 3] * x[:, j:j + 1]
+    rc, u, err = _device_call(N.SparseBlock3(rp, ci, blocks.reshape(-1)), q, np.full(nc, 0.4), r,
+                              1.0)
+    assert rc == 0 and np.isfinite(err)
+    np.testing.assert_array_equal(u, want.reshape(-1))
+    ci[rp[nc - 70] + 200] = nc
+    rc, u, err = _device_call(N.SparseBlock3(rp, ci, blocks.reshape(-1)), q, np.full(nc, 0.4), r,
+                              1.0)
+    assert rc == 0 and np.isnan(err) and np.isnan(u[3 * (nc - 70):3 * (nc - 69)]).all()
+    keep = np.repeat(np.arange(nc) != nc - 70, 3)
+    np.testing.assert_array_equal(u[keep], want.reshape(-1)[keep])
