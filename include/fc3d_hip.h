@@ -59,7 +59,9 @@ typedef struct fc3d_hip_params {
                                 start_trial_sweeps sweeps is below the zero
                                 start's; 3: the same against the resident
                                 reaction (previous time step)                   */
-  int schedule;              /* 0: autotuned; 1..10 explicit (7: single launch)   */
+  int schedule;              /* 0: autotuned (a small plain FP64 problem runs whole
+                                in one workgroup); 1..10 explicit (7: single
+                                launch; 10: several waves a slice)              */
   int sweeps_per_launch;     /* sweeps captured per graph replay (>=1); the FP64
                                 sweeps that end a precision = 1 solve replay at
                                 most 4 at a time                                 */
@@ -127,7 +129,8 @@ typedef struct fc3d_hip_stats {
   double sweep_kernel_ms;     /* instrumented: summed sweep-kernel durations    */
   int64_t sweep_kernel_launches;
   double sweep_kernel_bytes;  /* algorithmic bytes moved by those launches      */
-  int schedule;               /* sweep-kernel schedule used (autotuned when 0 given) */
+  int schedule;               /* sweep-kernel schedule used (autotuned when 0 given;
+                                 10 for the one-workgroup solve of a small problem) */
   /* warm_start = 2, 3: FP64 residual after one sweep from the fallback start
    * (zero, or the resident reaction) and from the learned start */
   double start_residual_fallback;
@@ -279,7 +282,8 @@ typedef struct fc3d_hip_batch_stats {
   int64_t total_sweeps;
   int64_t fp32_sweeps;
   double max_residual;
-  int schedule;               /* 1: one wave per problem, 2: four waves per problem */
+  int schedule;               /* 1: one wave per problem, 2: four waves per problem
+                                 (reactions in LDS up to 2048 contacts)         */
 } fc3d_hip_batch_stats;
 
 /* Problem p owns contacts [sum(nc[0..p)), sum(nc[0..p])) of the concatenated
