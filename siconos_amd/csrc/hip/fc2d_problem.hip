@@ -28,6 +28,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "fc2d_hip.h"
@@ -529,17 +530,25 @@ struct fc2d_hip_problem {
 constexpr int FC2D_GRAPH_SWEEPS = 16;
 
 // Builds Fc2dGroups for a problem in slot order (rows srp, places src, values
-// srv).  The order inside a colour is free: its contacts share no row entry.
+// srv), or nothing where its padded planes would not fit FC2D_LAYOUT_BYTES: the
+// solve then runs from the rows themselves.  The order inside a colour is free:
+// its contacts share no row entry.
+//
+// A group is as long as its longest row, so contacts that are all coupled to
+// each other (one large body touching m grains: a colour and a group of one
+// long lane each) take ~2 m^2 planes of 1280 bytes: 230 MB for m = 300, where
+// the rows take 4 MB, and 200 GB for 9200.  Up to the limit the layout is the
+// faster one there too (us a sweep, this / from the rows: 32 fully coupled
+// contacts 187 / 495, 200 of them 8900 / 18500; a body touching 200 of 8000
+// contacts 9000 / 18800): what draws the line is the memory, on the host while
+// it is built and on the device with the problem.
+constexpr int64_t FC2D_LAYOUT_BYTES = 256 << 20;
 static int build_groups(fc2d_hip_problem* h, const std::vector<int>& cptr,
                         const std::vector<int>& srp, const std::vector<int>& src,
                         const std::vector<double>& srv, const std::vector<double>& sdiag,
                         const std::vector<double>& sdet, const std::vector<double>& sq,
                         const std::vector<double>& smu) {
   const unsigned short zero = (unsigned short)(2 * h->nc);
-  std::vector<int> gptr(1, 0), slots;
-  std::vector<int2> planes;
-  std::vector<double> con, val;
-  std::vector<unsigned short> place;
   // entries of a row that the sweep adds: own-contact ones only as w * 0
   auto own = [&](int s, int e) { return src[(size_t)e] >> 1 == s; };
   auto row_len = [&](int s, int i) {
@@ -548,23 +557,33 @@ static int build_groups(fc2d_hip_problem* h, const std::vector<int>& cptr,
       n += h->own_zero || !own(s, e);
     return n;
   };
-  int np = 0;
+  // a colour's slots, longest rows first; then the groups and their planes
+  std::vector<std::pair<int, int>> m((size_t)h->nc);  // (-longest row, slot)
+  std::vector<int> gptr(1, 0);
+  std::vector<int2> planes;
+  int64_t np = 0;
+  for (int s = 0; s < h->nc; s++)
+    m[(size_t)s] = {-std::max(row_len(s, 0), row_len(s, 1)), s};
   for (int c = 0; c < h->ncolours; c++) {
-    std::vector<std::pair<int, int>> m;  // (-longest row, slot)
-    for (int s = cptr[(size_t)c]; s < cptr[(size_t)c + 1]; s++)
-      m.push_back({-std::max(row_len(s, 0), row_len(s, 1)), s});
-    std::sort(m.begin(), m.end());
-    for (size_t b = 0; b < m.size(); b += 64) {
-      const int k = -m[b].first;
-      const size_t g = planes.size();
-      planes.push_back(make_int2(np, k));
-      slots.resize(64 * (g + 1), -1);
-      con.resize(512 * (g + 1), 0.0);
-      place.resize((size_t)(np + k) * 128, zero);
-      val.resize((size_t)(np + k) * 128, 0.0);
-      for (size_t l = 0; l < 64 && b + l < m.size(); l++) {
-        const int s = m[b + l].second;
-        slots[64 * g + l] = s;
+    std::sort(m.begin() + cptr[(size_t)c], m.begin() + cptr[(size_t)c + 1]);
+    for (int b = cptr[(size_t)c]; b < cptr[(size_t)c + 1]; b += 64) {
+      const int k = -m[(size_t)b].first;
+      planes.push_back(make_int2((int)np, k));
+      np += k;
+    }
+    gptr.push_back((int)planes.size());
+  }
+  if (np * 128 * (int64_t)(sizeof(double) + sizeof(unsigned short)) > FC2D_LAYOUT_BYTES) return 0;
+  std::vector<int> slots(64 * planes.size(), -1);
+  std::vector<double> con(512 * planes.size(), 0.0), val((size_t)np * 128, 0.0);
+  std::vector<unsigned short> place((size_t)np * 128, zero);
+  size_t g = 0;
+  for (int c = 0; c < h->ncolours; c++) {
+    const int end = cptr[(size_t)c + 1];
+    for (int b = cptr[(size_t)c]; b < end; b += 64, g++) {
+      for (int l = 0; l < 64 && b + l < end; l++) {
+        const int s = m[(size_t)(b + l)].second;
+        slots[64 * g + (size_t)l] = s;
         double* cg = con.data() + 512 * g + l;
         for (int e = 0; e < 4; e++) cg[64 * e] = sdiag[4 * (size_t)s + (size_t)e];
         cg[256] = sdet[(size_t)s];
@@ -572,7 +591,7 @@ static int build_groups(fc2d_hip_problem* h, const std::vector<int>& cptr,
         cg[384] = sq[2 * (size_t)s + 1];
         cg[448] = smu[(size_t)s];
         for (int i = 0; i < 2; i++) {
-          size_t t = (size_t)np * 128 + (size_t)i * 64 + l;
+          size_t t = (size_t)planes[g].x * 128 + (size_t)i * 64 + (size_t)l;
           for (int e = srp[2 * (size_t)s + i]; e < srp[2 * (size_t)s + i + 1]; e++) {
             if (own(s, e) && !h->own_zero) continue;
             place[t] = own(s, e) ? zero : (unsigned short)src[(size_t)e];
@@ -581,9 +600,7 @@ static int build_groups(fc2d_hip_problem* h, const std::vector<int>& cptr,
           }
         }
       }
-      np += k;
     }
-    gptr.push_back((int)planes.size());
   }
   int rc;
   if ((rc = dev_upload(&h->g_ptr, gptr)) || (rc = dev_upload(&h->g_slot, slots)) ||
@@ -594,7 +611,7 @@ static int build_groups(fc2d_hip_problem* h, const std::vector<int>& cptr,
 }
 
 // The schedule a solve uses: the requested one, or automatically one workgroup
-// when the reactions fit its LDS (us a sweep, one workgroup / per colour: 31
+// when its LDS layout was built (us a sweep, one workgroup / per colour: 31
 // contacts 9.5 / 31, 431 15 / 47, 2070 19 / 62, 7056 40 / 71, 8985 49 / 73),
 // else one launch per colour when some colour holds more contacts than one
 // workgroup sweeps in two strides (below that, one workgroup's barriers cost
@@ -636,6 +653,123 @@ static int build_graph(fc2d_hip_problem* h) {
   if (e2 != hipSuccess) {
     h->graph = nullptr;
     set_error("fc2d graph instantiation: %s", hipGetErrorString(e2));
+    return NUMERICS_ERR_DEVICE;
+  }
+  return 0;
+}
+
+// Fills h from a checked problem; what it leaves behind on an error goes with h.
+static int build_problem(fc2d_hip_problem* h, int nc, const int64_t* row_ptr, const int64_t* cols,
+                         const double* vals, int row_mode, int own_zero, const double* diag,
+                         const double* q, const double* mu) {
+  int rc;
+  const int64_t n2 = 2 * (int64_t)nc, nnz = row_ptr[n2];
+  h->nc = nc;
+  h->row_mode = row_mode;
+  h->own_zero = own_zero ? 1 : 0;
+  double nq = 0.0;
+  for (int64_t i = 0; i < n2; i++) nq += q[i] * q[i];
+  h->norm_q = sqrt(nq);
+  if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
+      hipEventCreate(&h->ev[0]) != hipSuccess || hipEventCreate(&h->ev[1]) != hipSuccess) {
+    set_error("fc2d_hip_problem_create: stream or event creation failed");
+    return NUMERICS_ERR_DEVICE;
+  }
+  // conflict graph: contacts referenced by a row, symmetrised, without self
+  std::vector<std::vector<int>> nb((size_t)nc);
+  for (int c = 0; c < nc; c++)
+    for (int i = 0; i < 2; i++)
+      for (int64_t e = row_ptr[2 * c + i]; e < row_ptr[2 * c + i + 1]; e++) {
+        const int d = (int)(cols[e] >> 1);
+        if (d != c) {
+          nb[(size_t)c].push_back(d);
+          nb[(size_t)d].push_back(c);
+        }
+      }
+  std::vector<int> grp((size_t)nc + 1, 0), gci;
+  for (int c = 0; c < nc; c++) {
+    auto& v = nb[(size_t)c];
+    std::sort(v.begin(), v.end());
+    v.erase(std::unique(v.begin(), v.end()), v.end());
+    grp[(size_t)c + 1] = grp[(size_t)c] + (int)v.size();
+  }
+  gci.reserve((size_t)grp[(size_t)nc]);
+  for (int c = 0; c < nc; c++) gci.insert(gci.end(), nb[(size_t)c].begin(), nb[(size_t)c].end());
+  nb.clear();
+  int *d_rp = nullptr, *d_ci = nullptr, *d_col = nullptr;
+  std::vector<int> colour;
+  if ((rc = dev_upload(&d_rp, grp)) || (rc = dev_upload(&d_ci, gci)) ||
+      hipMalloc(&d_col, sizeof(int) * (size_t)nc) != hipSuccess) {
+    if (!rc) set_error("fc2d_hip_problem_create: allocation failed");
+    hipFree(d_rp);
+    hipFree(d_ci);
+    return rc ? rc : NUMERICS_ERR_DEVICE;
+  }
+  rc = fc3d::colour_on_device(nc, d_rp, d_ci, d_col, h->stream, &h->ncolours, &colour);
+  hipFree(d_rp);
+  hipFree(d_ci);
+  hipFree(d_col);
+  if (rc) return rc;
+  // colour-major order, index order inside a colour
+  std::vector<int> cptr((size_t)h->ncolours + 1, 0);
+  for (int c = 0; c < nc; c++) cptr[(size_t)colour[(size_t)c] + 1]++;
+  for (int k = 0; k < h->ncolours; k++) cptr[(size_t)k + 1] += cptr[(size_t)k];
+  h->order.assign((size_t)nc, 0);
+  h->slot.assign((size_t)nc, 0);
+  {
+    std::vector<int> fill(cptr.begin(), cptr.end() - 1);
+    for (int c = 0; c < nc; c++) {
+      const int s = fill[(size_t)colour[(size_t)c]]++;
+      h->order[(size_t)s] = c;
+      h->slot[(size_t)c] = s;
+    }
+  }
+  // rows, diagonal blocks, q, mu in slot order
+  std::vector<int> srp((size_t)n2 + 1, 0), src((size_t)(nnz ? nnz : 0));
+  std::vector<double> srv((size_t)(nnz ? nnz : 0)), sdiag(4 * (size_t)nc), sdet((size_t)nc),
+      sq((size_t)n2), smu((size_t)nc);
+  for (int s = 0; s < nc; s++) {
+    const int c = h->order[(size_t)s];
+    for (int i = 0; i < 2; i++) {
+      const int64_t row = 2 * (int64_t)c + i;
+      srp[2 * (size_t)s + i + 1] = (int)(row_ptr[row + 1] - row_ptr[row]);
+    }
+  }
+  for (int64_t i = 0; i < n2; i++) srp[(size_t)i + 1] += srp[(size_t)i];
+  for (int s = 0; s < nc; s++) {
+    const int c = h->order[(size_t)s];
+    for (int i = 0; i < 2; i++) {
+      const int64_t row = 2 * (int64_t)c + i;
+      int k = srp[2 * (size_t)s + i];
+      for (int64_t e = row_ptr[row]; e < row_ptr[row + 1]; e++, k++) {
+        const int d = (int)(cols[e] >> 1), comp = (int)(cols[e] & 1);
+        src[(size_t)k] = 2 * h->slot[(size_t)d] + comp;
+        srv[(size_t)k] = vals[e];
+      }
+      sq[2 * (size_t)s + i] = q[row];
+    }
+    for (int e = 0; e < 4; e++) sdiag[4 * (size_t)s + e] = diag[4 * (size_t)c + e];
+    // fc2d_nsgs.c:229-233
+    const double* B = diag + 4 * (size_t)c;
+    sdet[(size_t)s] = B[0] * B[3] - B[1] * B[2];
+    smu[(size_t)s] = mu[c];
+  }
+  std::vector<double> zero((size_t)n2, 0.0);
+  if ((rc = dev_upload(&h->cptr, cptr)) || (rc = dev_upload(&h->rp, srp)) ||
+      (rc = dev_upload(&h->rc, src)) || (rc = dev_upload(&h->rv, srv)) ||
+      (rc = dev_upload(&h->diag, sdiag)) || (rc = dev_upload(&h->det, sdet)) ||
+      (rc = dev_upload(&h->q, sq)) || (rc = dev_upload(&h->mu, smu)) ||
+      (rc = dev_upload(&h->r, zero)) || (rc = dev_upload(&h->u, zero)) ||
+      (rc = dev_upload(&h->light, std::vector<double>((size_t)nc, 0.0))))
+    return rc;
+  h->hcptr = cptr;
+  if (nc <= FC2D_LDS_CONTACTS &&
+      (rc = build_groups(h, cptr, srp, src, srv, sdiag, sdet, sq, smu)))
+    return rc;
+  if (hipMalloc(&h->err, sizeof(double)) != hipSuccess ||
+      hipMalloc(&h->out, sizeof(Fc2dOut)) != hipSuccess ||
+      hipMalloc(&h->st, sizeof(Fc2dState)) != hipSuccess) {
+    set_error("fc2d_hip_problem_create: allocation failed");
     return NUMERICS_ERR_DEVICE;
   }
   return 0;
@@ -696,127 +830,21 @@ int fc2d_hip_problem_create(int nc, const int64_t* row_ptr, const int64_t* cols,
       set_error("fc2d_hip_problem_create: column %lld out of range", (long long)cols[e]);
       return NUMERICS_ERR_INVALID_ARGUMENT;
     }
-  int rc = fc3d::use_device(device);
-  if (rc) return rc;
-  fc2d_hip_problem* h = new fc2d_hip_problem();
-  h->device = device;
-  h->nc = nc;
-  h->row_mode = row_mode;
-  h->own_zero = own_zero ? 1 : 0;
-  double nq = 0.0;
-  for (int64_t i = 0; i < n2; i++) nq += q[i] * q[i];
-  h->norm_q = sqrt(nq);
-  if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreate(&h->ev[0]) != hipSuccess || hipEventCreate(&h->ev[1]) != hipSuccess) {
-    set_error("fc2d_hip_problem_create: stream or event creation failed");
-    fc2d_hip_problem_destroy(h);
-    return NUMERICS_ERR_DEVICE;
+  const int rc0 = fc3d::use_device(device);
+  if (rc0) return rc0;
+  fc2d_hip_problem* h = nullptr;
+  int rc;
+  try {
+    h = new fc2d_hip_problem();
+    h->device = device;
+    rc = build_problem(h, nc, row_ptr, cols, vals, row_mode, own_zero, diag, q, mu);
+  } catch (const std::bad_alloc&) {
+    set_error("fc2d_hip_problem_create: out of host memory");
+    rc = NUMERICS_ERR_MEMORY;
   }
-  // conflict graph: contacts referenced by a row, symmetrised, without self
-  std::vector<std::vector<int>> nb((size_t)nc);
-  for (int c = 0; c < nc; c++)
-    for (int i = 0; i < 2; i++)
-      for (int64_t e = row_ptr[2 * c + i]; e < row_ptr[2 * c + i + 1]; e++) {
-        const int d = (int)(cols[e] >> 1);
-        if (d != c) {
-          nb[(size_t)c].push_back(d);
-          nb[(size_t)d].push_back(c);
-        }
-      }
-  std::vector<int> grp((size_t)nc + 1, 0), gci;
-  for (int c = 0; c < nc; c++) {
-    auto& v = nb[(size_t)c];
-    std::sort(v.begin(), v.end());
-    v.erase(std::unique(v.begin(), v.end()), v.end());
-    grp[(size_t)c + 1] = grp[(size_t)c] + (int)v.size();
-  }
-  gci.reserve((size_t)grp[(size_t)nc]);
-  for (int c = 0; c < nc; c++) gci.insert(gci.end(), nb[(size_t)c].begin(), nb[(size_t)c].end());
-  nb.clear();
-  int *d_rp = nullptr, *d_ci = nullptr, *d_col = nullptr;
-  std::vector<int> colour;
-  if ((rc = dev_upload(&d_rp, grp)) || (rc = dev_upload(&d_ci, gci)) ||
-      hipMalloc(&d_col, sizeof(int) * (size_t)nc) != hipSuccess) {
-    if (!rc) set_error("fc2d_hip_problem_create: allocation failed");
-    hipFree(d_rp);
-    hipFree(d_ci);
-    fc2d_hip_problem_destroy(h);
-    return rc ? rc : NUMERICS_ERR_DEVICE;
-  }
-  rc = fc3d::colour_on_device(nc, d_rp, d_ci, d_col, h->stream, &h->ncolours, &colour);
-  hipFree(d_rp);
-  hipFree(d_ci);
-  hipFree(d_col);
   if (rc) {
     fc2d_hip_problem_destroy(h);
     return rc;
-  }
-  // colour-major order, index order inside a colour
-  std::vector<int> cptr((size_t)h->ncolours + 1, 0);
-  for (int c = 0; c < nc; c++) cptr[(size_t)colour[(size_t)c] + 1]++;
-  for (int k = 0; k < h->ncolours; k++) cptr[(size_t)k + 1] += cptr[(size_t)k];
-  h->order.assign((size_t)nc, 0);
-  h->slot.assign((size_t)nc, 0);
-  {
-    std::vector<int> fill(cptr.begin(), cptr.end() - 1);
-    for (int c = 0; c < nc; c++) {
-      const int s = fill[(size_t)colour[(size_t)c]]++;
-      h->order[(size_t)s] = c;
-      h->slot[(size_t)c] = s;
-    }
-  }
-  // rows, diagonal blocks, q, mu in slot order
-  std::vector<int> srp((size_t)n2 + 1, 0), src((size_t)(nnz ? nnz : 0));
-  std::vector<double> srv((size_t)(nnz ? nnz : 0)), sdiag(4 * (size_t)nc), sdet((size_t)nc),
-      sq((size_t)n2), smu((size_t)nc);
-  for (int s = 0; s < nc; s++) {
-    const int c = h->order[(size_t)s];
-    for (int i = 0; i < 2; i++) {
-      const int64_t row = 2 * (int64_t)c + i;
-      srp[2 * (size_t)s + i + 1] = (int)(row_ptr[row + 1] - row_ptr[row]);
-    }
-  }
-  for (int64_t i = 0; i < n2; i++) srp[(size_t)i + 1] += srp[(size_t)i];
-  for (int s = 0; s < nc; s++) {
-    const int c = h->order[(size_t)s];
-    for (int i = 0; i < 2; i++) {
-      const int64_t row = 2 * (int64_t)c + i;
-      int k = srp[2 * (size_t)s + i];
-      for (int64_t e = row_ptr[row]; e < row_ptr[row + 1]; e++, k++) {
-        const int d = (int)(cols[e] >> 1), comp = (int)(cols[e] & 1);
-        src[(size_t)k] = 2 * h->slot[(size_t)d] + comp;
-        srv[(size_t)k] = vals[e];
-      }
-      sq[2 * (size_t)s + i] = q[row];
-    }
-    for (int e = 0; e < 4; e++) sdiag[4 * (size_t)s + e] = diag[4 * (size_t)c + e];
-    // fc2d_nsgs.c:229-233
-    const double* B = diag + 4 * (size_t)c;
-    sdet[(size_t)s] = B[0] * B[3] - B[1] * B[2];
-    smu[(size_t)s] = mu[c];
-  }
-  std::vector<double> zero((size_t)n2, 0.0);
-  if ((rc = dev_upload(&h->cptr, cptr)) || (rc = dev_upload(&h->rp, srp)) ||
-      (rc = dev_upload(&h->rc, src)) || (rc = dev_upload(&h->rv, srv)) ||
-      (rc = dev_upload(&h->diag, sdiag)) || (rc = dev_upload(&h->det, sdet)) ||
-      (rc = dev_upload(&h->q, sq)) || (rc = dev_upload(&h->mu, smu)) ||
-      (rc = dev_upload(&h->r, zero)) || (rc = dev_upload(&h->u, zero)) ||
-      (rc = dev_upload(&h->light, std::vector<double>((size_t)nc, 0.0)))) {
-    fc2d_hip_problem_destroy(h);
-    return rc;
-  }
-  h->hcptr = cptr;
-  if (nc <= FC2D_LDS_CONTACTS &&
-      (rc = build_groups(h, cptr, srp, src, srv, sdiag, sdet, sq, smu))) {
-    fc2d_hip_problem_destroy(h);
-    return rc;
-  }
-  if (hipMalloc(&h->err, sizeof(double)) != hipSuccess ||
-      hipMalloc(&h->out, sizeof(Fc2dOut)) != hipSuccess ||
-      hipMalloc(&h->st, sizeof(Fc2dState)) != hipSuccess) {
-    set_error("fc2d_hip_problem_create: allocation failed");
-    fc2d_hip_problem_destroy(h);
-    return NUMERICS_ERR_DEVICE;
   }
   *out = h;
   return 0;

@@ -264,3 +264,42 @@ def test_one_workgroup_at_the_edges_of_its_lds(lib, nc, row_mode, own_zero):
         out.append((P.reaction(), P.velocity(), s.iterations, s.residual, s.info))
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("nc", [200, 400])
+def test_fully_coupled_contacts(lib, nc):
+    """Contacts that are all coupled to each other, a colour each, on both
+    sides of the size whose padded layout is built: a problem takes little more
+    memory than its rows or the layout's bound, and both schedules give the
+    same bits."""
+    def free():  # (the HIP runtime that the library is linked to)
+        a, b = C.c_size_t(), C.c_size_t()
+        assert lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+    rng = np.random.default_rng(nc)
+    n2 = 2 * nc
+    G = rng.normal(size=(n2, n2)) / np.sqrt(n2)
+    W = G @ G.T + np.eye(n2)
+    rp = np.arange(n2 + 1, dtype=np.int64) * n2
+    cols = np.tile(np.arange(n2, dtype=np.int64), n2)
+    vals = np.ascontiguousarray(W.reshape(-1))
+    diag = np.concatenate([W[2 * c:2 * c + 2, 2 * c:2 * c + 2].reshape(-1, order="F")
+                           for c in range(nc)])
+    q, mu = rng.normal(size=n2), rng.uniform(0.1, 0.8, nc)
+    before = free()
+    h = C.c_void_p()
+    assert lib.fc2d_hip_problem_create(nc, N.lptr(rp), N.lptr(cols), N.dptr(vals), 0, 0,
+                                       N.dptr(diag), N.dptr(q), N.dptr(mu), 0,
+                                       C.byref(h)) == 0, capi.last_error()
+    P = N.Fc2dHipProblem.__new__(N.Fc2dHipProblem)
+    P._lib, P.nc, P._h = lib, nc, h
+    # 12 bytes an entry in the rows; the layout is kept up to 256 MB
+    assert before - free() < (12 * n2 * n2 + (256 << 20) + (32 << 20))
+    assert P.num_colours == nc
+    out = []
+    for schedule in (0, 2):
+        P.set_reaction(np.zeros(n2))
+        s = P.solve(max_iter=3, tol=1e-9, schedule=schedule)
+        out.append((P.reaction(), P.velocity(), s.iterations, s.residual, s.info))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
