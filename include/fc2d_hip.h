@@ -69,8 +69,8 @@ FC3D_API int fc2d_hip_get_velocity(fc2d_hip_problem* h, double* velocity);
  *     launch per colour, sweeps replayed from a captured graph;
  *   FC2D_SCHEDULE_AUTO: one workgroup up to 9200 contacts (its LDS then holds
  *     the reactions), unless its padded copy of the rows would take more than
- *     256 MB (hundreds of contacts all coupled to each other); else per colour when some colour holds more than
- *     2048 contacts, else one workgroup. */
+ *     256 MB (hundreds of contacts all coupled to each other); else per colour
+ *     when some colour holds more than 2048 contacts, else one workgroup. */
 enum { FC2D_SCHEDULE_AUTO = 0, FC2D_SCHEDULE_ONE_WORKGROUP = 1, FC2D_SCHEDULE_PER_COLOUR = 2 };
 
 typedef struct fc2d_hip_params {

@@ -283,7 +283,7 @@ typedef struct fc3d_hip_batch_stats {
   int64_t fp32_sweeps;
   double max_residual;
   int schedule;               /* 1: one wave per problem, 2: four waves per problem
-                                 (reactions in LDS up to 2048 contacts)         */
+                                 (reactions in LDS where that is the faster form) */
 } fc3d_hip_batch_stats;
 
 /* Problem p owns contacts [sum(nc[0..p)), sum(nc[0..p])) of the concatenated

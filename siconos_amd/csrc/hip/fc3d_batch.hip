@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "fc3d_batch.hpp"
+#include "fc3d_batch_rule.hpp"
 #include "fc3d_internal.hpp"
 #include "fc3d_layout.hpp"
 #include "fc3d_sweep.hpp"
@@ -245,8 +246,8 @@ __device__ __forceinline__ void reactions_out(const BatchArgs& A, const BatchPro
 // LDS: the problem's reactions live in LDS (32 bytes a contact, FP64 or FP32)
 // and the sweeps run in quads of waves (sweep_quads); HBM holds the reactions
 // before, after, and for the residual.  A launch lasts as long as its slowest
-// problem, whose colours are one or two slices, so the chain of a colour is
-// what counts: 1024 problems of 8-512 contacts, at most 1000 sweeps, 139 -> 100
+// problem, so the chain of a colour is what counts, where colours are one or
+// two slices (QuadRule; the wider ones keep a wave a slice): 1024 problems of 8-512 contacts, at most 1000 sweeps, 139 -> 100
 // ms in FP64 and 63 -> 51 mixed; 64 problems 104 -> 83 and 54 -> 46.
 template <int WPP, bool LDS, bool MIXED>
 __global__ __launch_bounds__(64 * WPP, WPP == 8 ? 1 : 2) void k_batch(
@@ -447,8 +448,10 @@ struct fc3d_hip_batch {
   float *vals32 = nullptr, *diag32 = nullptr, *q32 = nullptr, *mu32 = nullptr, *pli32 = nullptr;
   float4* r32 = nullptr;
   DevParams* prm = nullptr;
-  int *d_cbase = nullptr, max_nc = 0;
+  int* d_cbase = nullptr;
   unsigned short* d_ccol = nullptr;
+  QuadRule rule;
+  int lds_contacts = 0;  // the largest problem's contacts if quads sweep the batch, else 0
   mutable Transfer transfer;  // reactions and velocities in the caller's order
   int tuned_wpp[2] = {0, 0};
 };
@@ -539,10 +542,10 @@ static int ensure_fp32_batch(fc3d_hip_batch* b) {
 // Reactions in LDS, 32 bytes a contact: two workgroups' a CU (what the waves'
 // registers allow) within its 160 KB.
 constexpr int BATCH_LDS_CONTACTS = 2048;
-constexpr int BATCH_QUAD_PROBLEMS = 2048;
+constexpr int BATCH_WORKGROUPS_PER_CU = 2;
 
-// lds_contacts: the largest problem's contacts if the quads may keep the
-// reactions in LDS (four waves a problem), else 0.
+// lds_contacts: the largest problem's contacts if quads sweep the batch (four
+// waves a problem), else 0.
 static void launch_k_batch(const BatchArgs& A, const DevParams* prm, int wpp, int grid, int mixed,
                            int lds_contacts, hipStream_t s) {
   const dim3 g((unsigned)grid), t((unsigned)(64 * wpp));
@@ -588,10 +591,10 @@ static int launch_batch(fc3d_hip_batch* b, int wpp, int mixed) {
   FC3D_HIP_TRY(hipMemsetAsync(b->counter, 0, sizeof(int), b->stream));
   int cus = 0;
   FC3D_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
-  const int per_cu = wpp == 1 ? 8 : 2;  // 2 waves/SIMD at this kernel's register use
+  // 2 waves/SIMD at this kernel's register use
+  const int per_cu = wpp == 1 ? 8 : BATCH_WORKGROUPS_PER_CU;
   const int grid = std::max(1, std::min(b->nprob, cus * per_cu));
-  const int lds = b->max_nc <= BATCH_LDS_CONTACTS ? b->max_nc : 0;
-  launch_k_batch(batch_args(b), b->prm, wpp, grid, mixed, lds, b->stream);
+  launch_k_batch(batch_args(b), b->prm, wpp, grid, mixed, b->lds_contacts, b->stream);
   FC3D_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -694,8 +697,12 @@ int fc3d_hip_batch_create(int nprob, const int* nc, const int64_t* row_ptr,
   b->cptr = L.colour_slice_ptr;
   std::vector<int> cbase;
   std::vector<unsigned short> ccol;
-  b->max_nc = *std::max_element(b->nc.begin(), b->nc.end());
-  if (b->max_nc <= BATCH_LDS_CONTACTS) number_contacts(L, b->problems, &cbase, &ccol);
+  for (const BatchProblem& d : b->problems) b->rule.add(&b->cptr[(size_t)d.cptr_off], d.ncolours);
+  const int max_nc = *std::max_element(b->nc.begin(), b->nc.end());
+  if (max_nc <= BATCH_LDS_CONTACTS && b->rule.quads()) {
+    b->lds_contacts = max_nc;
+    number_contacts(L, b->problems, &cbase, &ccol);
+  }
   std::vector<int> order((size_t)nprob);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return nc[x] > nc[y]; });
@@ -832,12 +839,11 @@ int fc3d_hip_batch_solve(fc3d_hip_batch* b, const fc3d_hip_params* p, fc3d_hip_b
     set_error("fc3d_hip_batch_solve: schedule %d out of range [0, 2]", p->schedule);
     return NUMERICS_ERR_INVALID_ARGUMENT;
   }
-  // Few problems: quads, without the trial, whose 8 sweeps see the throughput
-  // of the start and not the slow problems that the launch ends with (it took
-  // one wave a problem where quads win).  ms one wave / quads, FP64: 1024
-  // problems 126 / 100, 2048 170 / 125, 4096 180 / 195; mixed: 68 / 51,
-  // 78 / 67, 97 / 99.
-  if (wpp == 0 && b->max_nc <= BATCH_LDS_CONTACTS && b->nprob <= BATCH_QUAD_PROBLEMS) wpp = 4;
+  if (wpp == 0 && b->lds_contacts) {
+    int cus = 1;
+    FC3D_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
+    if (b->rule.no_trial(b->nprob, BATCH_WORKGROUPS_PER_CU * cus, p->max_iter, p->tol)) wpp = 4;
+  }
   if (wpp == 0) {
     if (!b->tuned_wpp[mixed]) {
       double4* saved = nullptr;

@@ -161,3 +161,39 @@ def test_small_problem_in_one_workgroup(oracle, nc):
     s = P.solve(N.hip_params(tol=1e-5, max_iter=40))
     assert s.iterations == it
     np.testing.assert_array_equal(P.reaction(), ro)
+
+
+@pytest.mark.parametrize("kind", ["narrow", "wide"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_four_waves_in_both_forms(oracle, kind, precision):
+    """Colours of at most a slice up to the contacts that LDS holds (quads), and
+    colours of ten slices (four waves beside each other): four waves a problem
+    give the bits of one wave a problem, and in FP64 the oracle's."""
+    if kind == "narrow":  # 102 bodies: at most 51 contacts a colour
+        g = N.generate_random_pairs(102, 2048, 0.1, 0.9, 3)
+        probs = [(g.W, g.q, g.mu), (g.W, -0.5 * g.q, g.mu)]
+    else:  # a chain of contacts: two colours
+        rng = np.random.default_rng(4)
+        probs = []
+        for n in (1200, 65):
+            at = [[d for d in (c - 1, c, c + 1) if 0 <= d < n] for c in range(n)]
+            rp = np.concatenate([[0], np.cumsum([len(a) for a in at])])
+            blocks = [(3.0 if d == c else -0.4) * np.eye(3).reshape(-1)
+                      for c in range(n) for d in at[c]]
+            W = N.SparseBlock3(rp, np.concatenate(at), np.concatenate(blocks))
+            probs.append((W, rng.normal(size=3 * n), rng.uniform(0.2, 0.7, n)))
+    B = N.Batch(probs)
+    out = []
+    for schedule in (1, 2):
+        s, info, it, res = B.solve(N.hip_params(tol=1e-6, max_iter=12, warm_start=1,
+                                                schedule=schedule, precision=precision,
+                                                fp32_tol=1e-3))
+        out.append((B.reaction(), it))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    if precision == 0:
+        order = B.order()
+        for (W, q, mu), a, b, n in zip(probs, B.offsets[:-1], B.offsets[1:], out[0][1]):
+            _, ro, _, _, _ = oracle.nsgs(W, q, mu, tol=1e-30, max_iter=int(n),
+                                         order=order[a:b] - a)
+            np.testing.assert_array_equal(out[1][0][3 * a:3 * b], ro)
