@@ -17,6 +17,7 @@
 #include <cstring>
 #include <new>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "fc3d_internal.hpp"
@@ -76,14 +77,24 @@ __device__ inline void side_product(const double* __restrict__ g, const double* 
 // off the diagonal usually has one such pair, so the first pair found is
 // computed by every lane at its own addresses, without divergence; the
 // others (the diagonal's second side, two contacts between the same two
-// bodies, contacts with a body on both sides) follow in a loop.
-__global__ void k_asm_blocks(int64_t nnzb, const int* __restrict__ row, const int* __restrict__ col,
-                             const int* __restrict__ ba, const int* __restrict__ bb,
-                             const double* __restrict__ H, const double* __restrict__ G,
-                             double* __restrict__ W) {
+// bodies, contacts with a body on both sides) follow in a loop.  The block's
+// row is searched in the row pointers: a list of rows would be another array
+// to make on each call, and a small call is bound by such things.
+__global__ void k_asm_blocks(int nc, int64_t nnzb, const int64_t* __restrict__ rp,
+                             const int* __restrict__ col, const int* __restrict__ ba,
+                             const int* __restrict__ bb, const double* __restrict__ H,
+                             const double* __restrict__ G, double* __restrict__ W) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nnzb) return;
-  const int c = row[b], d = col[b];
+  int c = 0, end = nc;  // rp[c] <= b < rp[end]
+  while (end - c > 1) {
+    const int m = (c + end) >> 1;
+    if (rp[m] <= b)
+      c = m;
+    else
+      end = m;
+  }
+  const int d = col[b];
   const int kc[2] = {ba[c], bb[c]}, kd[2] = {ba[d], bb[d]};
   unsigned m = 0;
 #pragma unroll
@@ -121,13 +132,6 @@ __global__ void k_asm_q(int nc, const int* __restrict__ ba, const int* __restric
       for (int i = 0; i < 3; i++) s[i] += h[i + 3 * l] * vk[l];
   }
   for (int i = 0; i < 3; i++) q[3 * (size_t)c + i] = s[i];
-}
-
-// The row of every stored block, from the row pointers.
-__global__ void k_asm_rows(int nc, const int64_t* __restrict__ rp, int* __restrict__ row) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nc) return;
-  for (int64_t k = rp[c]; k < rp[c + 1]; k++) row[k] = c;
 }
 
 // fn(begin, end) over [0, n) in up to eight host threads (one per 16k rows).
@@ -172,16 +176,25 @@ static int merge_row(const int* a, int na, const int* b, int nb, int c, T* out) 
   return n;
 }
 
-// RAII device buffers
+// The call's device arrays, parts of one allocation (a call on 100 contacts,
+// which its copies, allocations and launches make up: 225 us with one each,
+// 212 so).
 struct AsmBufs {
-  std::vector<void*> p;
+  std::vector<std::pair<void**, size_t>> parts;  // pointer to set, place
+  size_t bytes = 0;
+  char* p = nullptr;
   ~AsmBufs() {
-    for (void* x : p) hipFree(x);
+    if (p) hipFree(p);
   }
   template <typename T>
-  hipError_t get(T** out, size_t n) {
-    hipError_t e = hipMalloc(out, sizeof(T) * (n ? n : 1));
-    if (e == hipSuccess) p.push_back(*out);
+  void want(T** out, size_t n) {
+    parts.push_back({(void**)out, bytes});
+    bytes += (sizeof(T) * n + 255) / 256 * 256;
+  }
+  hipError_t get() {
+    const hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipSuccess)
+      for (const auto& x : parts) *x.first = p + x.second;
     return e;
   }
 };
@@ -198,21 +211,21 @@ static int assemble_values(int nbodies, int nc, const int* body_a, const int* bo
                            double* device_ms) {
   const int64_t nnzb = out->nnzb;
   AsmBufs B;
-  int *d_ba, *d_bb, *d_row, *d_col;
+  int *d_ba, *d_bb, *d_col;
   int64_t* d_rp;
   double *d_H, *d_M, *d_v, *d_G, *d_W, *d_q;
   const size_t mlen = (size_t)nbodies * (minv_diagonal ? 6 : 36);
-  FC3D_HIP_TRY(B.get(&d_ba, (size_t)nc));
-  FC3D_HIP_TRY(B.get(&d_bb, (size_t)nc));
-  FC3D_HIP_TRY(B.get(&d_row, (size_t)nnzb));
-  FC3D_HIP_TRY(B.get(&d_rp, (size_t)nc + 1));
-  FC3D_HIP_TRY(B.get(&d_col, (size_t)nnzb));
-  FC3D_HIP_TRY(B.get(&d_H, 36 * (size_t)nc));
-  FC3D_HIP_TRY(B.get(&d_M, mlen));
-  FC3D_HIP_TRY(B.get(&d_v, 6 * (size_t)nbodies));
-  FC3D_HIP_TRY(B.get(&d_G, 36 * (size_t)nc));
-  FC3D_HIP_TRY(B.get(&d_W, 9 * (size_t)nnzb));
-  FC3D_HIP_TRY(B.get(&d_q, 3 * (size_t)nc));
+  B.want(&d_ba, (size_t)nc);
+  B.want(&d_bb, (size_t)nc);
+  B.want(&d_rp, (size_t)nc + 1);
+  B.want(&d_col, (size_t)nnzb);
+  B.want(&d_H, 36 * (size_t)nc);
+  B.want(&d_M, mlen);
+  B.want(&d_v, 6 * (size_t)nbodies);
+  B.want(&d_G, 36 * (size_t)nc);
+  B.want(&d_W, 9 * (size_t)nnzb);
+  B.want(&d_q, 3 * (size_t)nc);
+  FC3D_HIP_TRY(B.get());
   FC3D_HIP_TRY(hipMemcpy(d_ba, body_a, sizeof(int) * (size_t)nc, hipMemcpyHostToDevice));
   FC3D_HIP_TRY(hipMemcpy(d_bb, body_b, sizeof(int) * (size_t)nc, hipMemcpyHostToDevice));
   FC3D_HIP_TRY(hipMemcpy(d_rp, out->row_ptr, sizeof(int64_t) * ((size_t)nc + 1),
@@ -226,14 +239,12 @@ static int assemble_values(int nbodies, int nc, const int* body_a, const int* bo
   FC3D_HIP_TRY(hipEventCreate(&e0));
   FC3D_HIP_TRY(hipEventCreate(&e1));
   FC3D_HIP_TRY(hipEventRecord(e0, 0));
-  hipLaunchKernelGGL(k_asm_rows, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, 0, nc,
-                     (const int64_t*)d_rp, d_row);
   hipLaunchKernelGGL(k_asm_g, dim3((unsigned)((2 * (size_t)nc + 255) / 256)), dim3(256), 0, 0, nc,
                      (const int*)d_ba, (const int*)d_bb, (const double*)d_H, (const double*)d_M,
                      minv_diagonal ? 1 : 0, d_G);
-  hipLaunchKernelGGL(k_asm_blocks, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, nnzb,
-                     (const int*)d_row, (const int*)d_col, (const int*)d_ba, (const int*)d_bb,
-                     (const double*)d_H, (const double*)d_G, d_W);
+  hipLaunchKernelGGL(k_asm_blocks, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, nc,
+                     nnzb, (const int64_t*)d_rp, (const int*)d_col, (const int*)d_ba,
+                     (const int*)d_bb, (const double*)d_H, (const double*)d_G, d_W);
   hipLaunchKernelGGL(k_asm_q, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, 0, nc,
                      (const int*)d_ba, (const int*)d_bb, (const double*)d_H, (const double*)d_v,
                      d_q);
