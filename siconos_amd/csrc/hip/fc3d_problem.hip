@@ -650,6 +650,7 @@ struct fc3d_hip_problem {
   int* d_cbase = nullptr;
   unsigned short* d_ccol = nullptr;
   SmallSolve* d_small = nullptr;
+  hipEvent_t small_ev[2] = {nullptr, nullptr};
   // device
   int *len = nullptr, *dpos = nullptr, *koff = nullptr, *kmax = nullptr, *col = nullptr;
   double *vals = nullptr, *diag = nullptr, *q = nullptr, *mu = nullptr, *pli = nullptr;
@@ -1625,8 +1626,11 @@ static int tune_schedule(fc3d_hip_problem* h, int phase, double norm_q, double l
 }
 
 // A small problem's plain FP64 solve runs whole in one workgroup (k_batch's
-// quads, reactions in LDS; the same sweeps and bits): no launch, no memory
-// round trip for a colour's reactions.  The two quads take a colour's slices
+// quads, reactions in LDS): no launch, no memory round trip for a colour's
+// reactions.  After as many sweeps its reactions are those of the launches per
+// colour bit for bit; the light error and the residual, which end the solve,
+// are added per lane and then over the eight waves instead of slice by slice,
+// so their last bits differ.  The two quads take a colour's slices
 // side by side, so it pays to three slices a colour.  us a sweep, this /
 // launches per colour: 40 contacts 47 / 75, 200 90 / 115, 500 (two slices)
 // 84 / 113, 1000 (three) 133 / 145 and 117 / 115, 1500 (four, five) 180 / 161
@@ -1641,24 +1645,21 @@ static bool small_solve(const fc3d_hip_problem* h, const fc3d_hip_params* p, boo
 
 static int solve_small(fc3d_hip_problem* h, const fc3d_hip_params* p, fc3d_hip_stats* s) {
   int rc;
-  hipEvent_t t0, t1;
   SmallSolve x;
   std::memset(&x, 0, sizeof x);
   x.problem = {0, h->ncolours, 0, h->nslices, h->norm_q};
   FC3D_HIP_TRY(hipMemcpyAsync(h->d_small, &x, sizeof x, hipMemcpyHostToDevice, h->stream));
-  FC3D_HIP_TRY(hipEventCreate(&t0));
-  FC3D_HIP_TRY(hipEventCreate(&t1));
-  FC3D_HIP_TRY(hipEventRecord(t0, h->stream));
+  for (hipEvent_t& e : h->small_ev)
+    if (!e) FC3D_HIP_TRY(hipEventCreate(&e));
+  FC3D_HIP_TRY(hipEventRecord(h->small_ev[0], h->stream));
   if ((rc = launch_small_solve(ptrs64(h, h->part), h->d_cps, h->d_cbase, h->d_ccol, h->nc, h->prm,
                                h->d_small, h->stream)))
     return rc;
-  FC3D_HIP_TRY(hipEventRecord(t1, h->stream));
+  FC3D_HIP_TRY(hipEventRecord(h->small_ev[1], h->stream));
   FC3D_HIP_TRY(hipMemcpyAsync(&x, h->d_small, sizeof x, hipMemcpyDeviceToHost, h->stream));
   FC3D_HIP_TRY(hipStreamSynchronize(h->stream));
   float ms = 0.f;
-  hipEventElapsedTime(&ms, t0, t1);
-  hipEventDestroy(t0);
-  hipEventDestroy(t1);
+  hipEventElapsedTime(&ms, h->small_ev[0], h->small_ev[1]);
   s->solve_ms = ms;
   s->iterations = x.iterations;
   s->incr_error = x.incr;
@@ -1908,6 +1909,8 @@ void fc3d_hip_problem_destroy(fc3d_hip_problem* h) {
   free_accel(h);
   free_stage_bufs(h);
   h->transfer.release();
+  for (hipEvent_t e : h->small_ev)
+    if (e) hipEventDestroy(e);
   void* dfp[] = {h->dep_ptr, h->dep_idx, h->qlist, h->done,    h->df,    h->d_block_dst,
                  h->d_o2s,    h->d_cps,    h->d_planes, h->d_cbase, h->d_ccol, h->d_small,   h->d_ba,   h->d_bb,   h->d_inc_ptr, h->d_inc, h->d_H,
                  h->d_minv,   h->d_vfree,  h->d_V,    h->d_H32,     h->d_minv32, h->d_V32,
