@@ -637,7 +637,7 @@ __device__ int nsn_newton_std_fp32(const LocalProblem<T>& lp, T* r, const LocalP
   return 1;
 }
 
-// sqrt(x) / d < t or <= t (with `equal`), the root and the quotient taken only
+// sqrt(x) / d < t (or <= t) for td = t d, the root and the quotient taken only
 // where the squares do not decide: these tests are mostly orders of magnitude
 // off their threshold.  x and (t d)^2 carry a few ulp each, so when they are a
 // factor 1 +- 1e-9 apart they order as the rounded sides do; t d > 1e-140 and
@@ -829,6 +829,9 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
     if (!damped && P.formulation != 1)
       return nsn_newton_std_fp32<T>(lp, r, P, tol, rho, residual);
   }
+  // (in double only the Jean-Moreau formulation comes here: STD has
+  // nsn_newton_std_fp64)
+  const int formulation = sizeof(T) == 8 ? 1 : P.formulation;
   const T nq = qsqrt<T>(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
   T nrel = T(1);
   if (nq > num<T>::eps) nrel = qdiv<T>(nrel, nq);
@@ -839,11 +842,11 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
   T B[9] = {T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
   local_velocity<T>(lp, r, v);
   T t = T(1);
-  ac_function<T, false>(P.formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
+  ac_function<T, false>(formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
   *residual = qsqrt<T>(F[0] * F[0] + F[1] * F[1] + F[2] * F[2]) * nrel;
   if (*residual < tol) return 0;
   for (int inew = 1; inew < P.newton_max_iter; ++inew) {
-    ac_function<T, true>(P.formulation, r, v, lp.mu, rho, F, A, B);
+    ac_function<T, true>(formulation, r, v, lp.mu, rho, F, A, B);
     T AW[9];
     mm3x3<T>(A, lp.W, AW);
     T M[9], d[3];
@@ -879,7 +882,7 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
     if (damped) {
       if (!info3) {
         T t_opt = T(1);
-        line_search_gp<T>(lp, P.formulation, &t_opt, r, dR, rho, P.ls_max_iter, F, A, B, v);
+        line_search_gp<T>(lp, formulation, &t_opt, r, dR, rho, P.ls_max_iter, F, A, B, v);
         t = t_opt;
       }
       r[0] = r[0] + t * dR[0];
@@ -889,7 +892,7 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
       r[0] += dR[0]; r[1] += dR[1]; r[2] += dR[2];
     }
     local_velocity<T>(lp, r, v);
-    ac_function<T, false>(P.formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
+    ac_function<T, false>(formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
     *residual = qsqrt<T>(F[0] * F[0] + F[1] * F[1] + F[2] * F[2]) * nrel;
     const T ndR = qsqrt<T>(dR[0] * dR[0] + dR[1] * dR[1] + dR[2] * dR[2]);
     if (damped) {
@@ -1089,11 +1092,13 @@ __device__ int local_solve(const LocalProblem<T>& lp, T* r, const LocalParams& P
     *residual = T(0);
     return 0;
   }
-  if constexpr (sizeof(T) == 8)
+  if constexpr (sizeof(T) == 8) {
     return newton_solvers_fp64(lp, r, P, tol, state_pli, rho, residual);
-  if (P.solver == 550) return nsn_newton<T>(lp, r, P, tol, rho, false, residual);
-  if (P.solver == 551) return nsn_newton<T>(lp, r, P, tol, rho, true, residual);
-  return hybrid_solve<T>(lp, r, P, tol, state_pli, rho, residual);
+  } else {
+    if (P.solver == 550) return nsn_newton<T>(lp, r, P, tol, rho, false, residual);
+    if (P.solver == 551) return nsn_newton<T>(lp, r, P, tol, rho, true, residual);
+    return hybrid_solve<T>(lp, r, P, tol, state_pli, rho, residual);
+  }
 }
 
 }  // namespace fc3d
