@@ -45,7 +45,7 @@ class _Hip:
         self.bufs = []
 
 
-def _device_call(W, q, mu, r, norm):
+def _device_call(W, q, mu, r, norm, nnzb=None):
     d = _Hip()
     try:
         u0 = np.full(3 * W.nc, -1.0)
@@ -56,8 +56,8 @@ def _device_call(W, q, mu, r, norm):
                 d.upload(np.asarray(q, dtype=np.float64)), d.upload(np.asarray(mu, dtype=np.float64)),
                 d.upload(np.asarray(r, dtype=np.float64))]
         pu, pe = d.upload(u0), d.upload(e0)
-        rc = capi.load().fc3d_hip_compute_error_device(W.nc, int(W.nnzb), *ptrs, norm, pu, pe, 0,
-                                                       None)
+        rc = capi.load().fc3d_hip_compute_error_device(
+            W.nc, int(W.nnzb) if nnzb is None else nnzb, *ptrs, norm, pu, pe, 0, None)
         u = d.download(pu, u0)
         e = d.download(pe, e0)
         return rc, u, float(e[0])
@@ -126,12 +126,8 @@ def test_no_alloc_residual_rows_of_every_length(nc):
     np.testing.assert_array_equal(u[keep], want.reshape(-1)[keep])
     past = W.row_ptr.copy()
     past[nc] += 1
-    short = N.SparseBlock3(past, ci, blocks.reshape(-1))
-    type(short).nnzb = property(lambda s: int(rp[-1]))
-    try:
-        rc, u, err = _device_call(short, q, np.full(nc, 0.4), r, 1.0)
-    finally:
-        type(short).nnzb = property(lambda s: int(s.row_ptr[-1]))
+    rc, u, err = _device_call(N.SparseBlock3(past, ci, blocks.reshape(-1)), q, np.full(nc, 0.4),
+                              r, 1.0, nnzb=int(rp[-1]))
     assert rc == 0 and np.isnan(err) and np.isnan(u[-3:]).all()
     np.testing.assert_array_equal(u[:-3], want.reshape(-1)[:-3])
 
@@ -140,7 +136,10 @@ def test_no_alloc_residual_rows_of_every_length(nc):
 def test_no_alloc_residual_on_both_sides_of_its_wide_form(nc):
     """The largest problem that takes four waves per 64 contacts and one that
     takes one wave, its last wave ragged: rows of 0 to 7 blocks and one of 300,
-    then a column out of range."""
+    then a column out of range, then row pointers that reach past the end and
+    fall back, in a wave that has others after it in its workgroup: those two
+    rows are NaN, and all others keep their bits, the wave's own too, which it
+    walks from memory."""
     rng = np.random.default_rng(nc)
     per = rng.integers(0, 8, nc)
     per[nc - 70] = 300
@@ -164,4 +163,14 @@ def test_no_alloc_residual_on_both_sides_of_its_wide_form(nc):
                               1.0)
     assert rc == 0 and np.isnan(err) and np.isnan(u[3 * (nc - 70):3 * (nc - 69)]).all()
     keep = np.repeat(np.arange(nc) != nc - 70, 3)
+    np.testing.assert_array_equal(u[keep], want.reshape(-1)[keep])
+    ci[rp[nc - 70] + 200] = 0
+    row = 64 * 4 * 17 + 64 + 20  # lane 20 of the second wave of a workgroup of four
+    out = rp.copy()
+    out[row + 1] = rp[-1] + 1
+    rc, u, err = _device_call(N.SparseBlock3(out, ci, blocks.reshape(-1)), q, np.full(nc, 0.4), r,
+                              1.0, nnzb=int(rp[-1]))
+    keep = np.repeat(~np.isin(np.arange(nc), (row, row + 1, nc - 70)), 3)
+    bad = slice(3 * row, 3 * (row + 2))
+    assert rc == 0 and np.isnan(err) and np.isnan(u[bad]).all()
     np.testing.assert_array_equal(u[keep], want.reshape(-1)[keep])
