@@ -84,16 +84,26 @@ __global__ void k_asm_blocks(int nc, int64_t nnzb, const int64_t* __restrict__ r
                              const int* __restrict__ col, const int* __restrict__ ba,
                              const int* __restrict__ bb, const double* __restrict__ H,
                              const double* __restrict__ G, double* __restrict__ W) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int64_t b0 =
+      (int64_t)blockIdx.x * blockDim.x + __builtin_amdgcn_readfirstlane(threadIdx.x - lane);
+  const int64_t b = b0 + lane;
   if (b >= nnzb) return;
-  int c = 0, end = nc;  // rp[c] <= b < rp[end]
-  while (end - c > 1) {
-    const int m = (c + end) >> 1;
-    if (rp[m] <= b)
-      c = m;
-    else
-      end = m;
-  }
+  // rp[c] <= b < rp[end]: for the wave's first block (scalar loads), then from
+  // there, a row holding at least one block
+  auto search = [&](int64_t k, int& c, int& end) {
+    while (end - c > 1) {
+      const int m = (c + end) >> 1;
+      if (rp[m] <= k)
+        c = m;
+      else
+        end = m;
+    }
+  };
+  int c = 0, end = nc;
+  search(b0, c, end);
+  end = min(c + 64, nc);
+  search(b, c, end);
   const int d = col[b];
   const int kc[2] = {ba[c], bb[c]}, kd[2] = {ba[d], bb[d]};
   unsigned m = 0;
