@@ -829,9 +829,8 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
     if (!damped && P.formulation != 1)
       return nsn_newton_std_fp32<T>(lp, r, P, tol, rho, residual);
   }
-  // (in double only the Jean-Moreau formulation comes here: STD has
-  // nsn_newton_std_fp64)
-  const int formulation = sizeof(T) == 8 ? 1 : P.formulation;
+  // (in double only the Jean-Moreau formulation comes here, STD having
+  // nsn_newton_std_fp64; inlined behind that test the rest is dropped)
   const T nq = qsqrt<T>(lp.q[0] * lp.q[0] + lp.q[1] * lp.q[1] + lp.q[2] * lp.q[2]);
   T nrel = T(1);
   if (nq > num<T>::eps) nrel = qdiv<T>(nrel, nq);
@@ -842,11 +841,11 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
   T B[9] = {T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
   local_velocity<T>(lp, r, v);
   T t = T(1);
-  ac_function<T, false>(formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
+  ac_function<T, false>(P.formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
   *residual = qsqrt<T>(F[0] * F[0] + F[1] * F[1] + F[2] * F[2]) * nrel;
   if (*residual < tol) return 0;
   for (int inew = 1; inew < P.newton_max_iter; ++inew) {
-    ac_function<T, true>(formulation, r, v, lp.mu, rho, F, A, B);
+    ac_function<T, true>(P.formulation, r, v, lp.mu, rho, F, A, B);
     T AW[9];
     mm3x3<T>(A, lp.W, AW);
     T M[9], d[3];
@@ -882,7 +881,7 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
     if (damped) {
       if (!info3) {
         T t_opt = T(1);
-        line_search_gp<T>(lp, formulation, &t_opt, r, dR, rho, P.ls_max_iter, F, A, B, v);
+        line_search_gp<T>(lp, P.formulation, &t_opt, r, dR, rho, P.ls_max_iter, F, A, B, v);
         t = t_opt;
       }
       r[0] = r[0] + t * dR[0];
@@ -892,7 +891,7 @@ __device__ int nsn_newton(const LocalProblem<T>& lp, T* r, const LocalParams& P,
       r[0] += dR[0]; r[1] += dR[1]; r[2] += dR[2];
     }
     local_velocity<T>(lp, r, v);
-    ac_function<T, false>(formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
+    ac_function<T, false>(P.formulation, r, v, lp.mu, rho, F, nullptr, nullptr);
     *residual = qsqrt<T>(F[0] * F[0] + F[1] * F[1] + F[2] * F[2]) * nrel;
     const T ndR = qsqrt<T>(dR[0] * dR[0] + dR[1] * dR[1] + dR[2] * dR[2]);
     if (damped) {
