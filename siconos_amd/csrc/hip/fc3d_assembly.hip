@@ -24,12 +24,17 @@
 
 namespace fc3d {
 
+// A contact's two threads also write down its blocks' row, for k_asm_blocks: as
+// a kernel of its own that took 13 us at 200k contacts, as a search in the row
+// pointers by every wave of k_asm_blocks 20 us (70 at 1M).
 __global__ void k_asm_g(int nc, const int* __restrict__ ba, const int* __restrict__ bb,
                         const double* __restrict__ H, const double* __restrict__ Minv, int diag,
-                        double* __restrict__ G) {
+                        const int64_t* __restrict__ rp, double* __restrict__ G,
+                        int* __restrict__ row) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= 2 * nc) return;
   const int c = t >> 1, side = t & 1;
+  for (int64_t k = rp[c] + side; k < rp[c + 1]; k += 2) row[k] = c;
   const int k = side ? bb[c] : ba[c];
   const double* h = H + 36 * (size_t)c + 18 * side;
   double* g = G + 36 * (size_t)c + 18 * side;
@@ -77,34 +82,14 @@ __device__ inline void side_product(const double* __restrict__ g, const double* 
 // off the diagonal usually has one such pair, so the first pair found is
 // computed by every lane at its own addresses, without divergence; the
 // others (the diagonal's second side, two contacts between the same two
-// bodies, contacts with a body on both sides) follow in a loop.  The block's
-// row is searched in the row pointers: a list of rows would be another array
-// to make on each call, and a small call is bound by such things.
-__global__ void k_asm_blocks(int nc, int64_t nnzb, const int64_t* __restrict__ rp,
-                             const int* __restrict__ col, const int* __restrict__ ba,
-                             const int* __restrict__ bb, const double* __restrict__ H,
-                             const double* __restrict__ G, double* __restrict__ W) {
-  const int lane = threadIdx.x & 63;
-  const int64_t b0 =
-      (int64_t)blockIdx.x * blockDim.x + __builtin_amdgcn_readfirstlane(threadIdx.x - lane);
-  const int64_t b = b0 + lane;
+// bodies, contacts with a body on both sides) follow in a loop.
+__global__ void k_asm_blocks(int64_t nnzb, const int* __restrict__ row, const int* __restrict__ col,
+                             const int* __restrict__ ba, const int* __restrict__ bb,
+                             const double* __restrict__ H, const double* __restrict__ G,
+                             double* __restrict__ W) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nnzb) return;
-  // rp[c] <= b < rp[end]: for the wave's first block (scalar loads), then from
-  // there, a row holding at least one block
-  auto search = [&](int64_t k, int& c, int& end) {
-    while (end - c > 1) {
-      const int m = (c + end) >> 1;
-      if (rp[m] <= k)
-        c = m;
-      else
-        end = m;
-    }
-  };
-  int c = 0, end = nc;
-  search(b0, c, end);
-  end = min(c + 64, nc);
-  search(b, c, end);
-  const int d = col[b];
+  const int c = row[b], d = col[b];
   const int kc[2] = {ba[c], bb[c]}, kd[2] = {ba[d], bb[d]};
   unsigned m = 0;
 #pragma unroll
@@ -221,13 +206,14 @@ static int assemble_values(int nbodies, int nc, const int* body_a, const int* bo
                            double* device_ms) {
   const int64_t nnzb = out->nnzb;
   AsmBufs B;
-  int *d_ba, *d_bb, *d_col;
+  int *d_ba, *d_bb, *d_row, *d_col;
   int64_t* d_rp;
   double *d_H, *d_M, *d_v, *d_G, *d_W, *d_q;
   const size_t mlen = (size_t)nbodies * (minv_diagonal ? 6 : 36);
   B.want(&d_ba, (size_t)nc);
   B.want(&d_bb, (size_t)nc);
   B.want(&d_rp, (size_t)nc + 1);
+  B.want(&d_row, (size_t)nnzb);
   B.want(&d_col, (size_t)nnzb);
   B.want(&d_H, 36 * (size_t)nc);
   B.want(&d_M, mlen);
@@ -251,10 +237,10 @@ static int assemble_values(int nbodies, int nc, const int* body_a, const int* bo
   FC3D_HIP_TRY(hipEventRecord(e0, 0));
   hipLaunchKernelGGL(k_asm_g, dim3((unsigned)((2 * (size_t)nc + 255) / 256)), dim3(256), 0, 0, nc,
                      (const int*)d_ba, (const int*)d_bb, (const double*)d_H, (const double*)d_M,
-                     minv_diagonal ? 1 : 0, d_G);
-  hipLaunchKernelGGL(k_asm_blocks, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, nc,
-                     nnzb, (const int64_t*)d_rp, (const int*)d_col, (const int*)d_ba,
-                     (const int*)d_bb, (const double*)d_H, (const double*)d_G, d_W);
+                     minv_diagonal ? 1 : 0, (const int64_t*)d_rp, d_G, d_row);
+  hipLaunchKernelGGL(k_asm_blocks, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, nnzb,
+                     (const int*)d_row, (const int*)d_col, (const int*)d_ba, (const int*)d_bb,
+                     (const double*)d_H, (const double*)d_G, d_W);
   hipLaunchKernelGGL(k_asm_q, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, 0, nc,
                      (const int*)d_ba, (const int*)d_bb, (const double*)d_H, (const double*)d_v,
                      d_q);
