@@ -114,9 +114,10 @@ def test_full_4096_problem_launch_converges_everywhere(oracle, batch4096, precis
 @pytest.mark.parametrize("sizes", [(1, 2), (63, 64, 65), (513, 40), (2048, 8), (2049, 8)])
 @pytest.mark.parametrize("mode", [1, 2])
 def test_quads_at_their_edges(oracle, sizes, mode):
-    """Four waves a problem at the edges of a slice, of the reactions' place in
-    LDS (2048 contacts) and beyond it, with rows longer than the 16 planes a
-    lane holds, bit for bit per problem."""
+    """Four waves a problem at the edges of a slice, with rows longer than the 16
+    planes a lane holds, and around the 2048 contacts that LDS holds (here in
+    colours of three slices, so a wave a slice; test_four_waves_in_both_forms
+    has 2048 contacts in LDS), bit for bit per problem."""
     probs = []
     for k, n in enumerate(sizes):
         nb = max(3, n // 6)  # ~24 blocks a row
